@@ -1,0 +1,47 @@
+"""The fast repeats of k_eos against its general form.
+
+Waves whose elements lie strictly between eosvmin and eosvmax run a form
+without those cases; pmin = -0.0 makes every wave take the general form (its
+clamp gives the same values up to the sign of zero).  With limits that cut
+through the elements' volumes a mesh holds waves of both kinds.
+"""
+import numpy as np
+import pytest
+
+import lulesh_amd as la
+from helpers import context_from_oracle, max_rel, upload_state
+from oracle_binding import OracleDomain
+
+pytestmark = pytest.mark.gpu
+
+FIELDS = ["e", "p", "q", "ss", "v"]
+# FP64 keeps the reference's rounding in both forms; the other two may fuse
+# their multiply-adds differently in each (bounds of the forms' own tests)
+TOLERANCE = {la.FP64: 0.0, la.FP64_FMA: 1e-11, la.MIXED: 1e-5}
+
+
+@pytest.mark.parametrize("precision", sorted(TOLERANCE))
+@pytest.mark.parametrize("eosvmin,eosvmax", [(1e-9, 1e9), (0.0, 1e9), (1e-9, 1.0), (0.95, 1.01), (0.0, 0.0)])
+def test_waves_between_the_volume_limits(precision, eosvmin, eosvmax):
+    o = OracleDomain(12, 11, 1, 1)
+    for _ in range(40):
+        o.call("time_increment")
+        assert o.call("lagrange_leapfrog") == 0
+    runs = []
+    for pmin in (0.0, -0.0):
+        k = la.default_constants()
+        k.eosvmin, k.eosvmax, k.pmin = eosvmin, eosvmax, pmin
+        ctx = context_from_oracle(o, precision=precision, constants=k)
+        upload_state(ctx, o)
+        dt = o.get("deltatime")
+        assert ctx.lagrange_nodal(dt) == 0
+        assert ctx.lagrange_elements(dt) == 0
+        status, courant, hydro = ctx.time_constraints()
+        assert status == 0
+        runs.append(({f: ctx.download(f) for f in FIELDS}, courant, hydro))
+    (fast, c0, h0), (general, c1, h1) = runs
+    for f in FIELDS:
+        assert np.all(np.isfinite(fast[f])), f
+        assert max_rel(fast[f], general[f]) <= TOLERANCE[precision], f
+    assert abs(c0 - c1) <= TOLERANCE[precision] * abs(c1)
+    assert h0 == h1
