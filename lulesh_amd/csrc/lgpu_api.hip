@@ -237,7 +237,8 @@ int set_eos_order(lgpu_ctx *c, int k)
          for (int j = 0; j < k && r < rest.size(); ++j) order.push_back(rest[r++]);
       }
    }
-   const std::vector<EosSlot> slots = eos_slots(order, c->hostRegStart, c->hostRegRep, c->numElem);
+   const std::vector<EosSlot> slots = eos_slots(order, c->hostRegStart, c->hostRegRep, c->numElem,
+                                               c->s.eosShare);
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
    HIP_OR_RETURN(c, hipMemcpy(const_cast<EosSlot *>(c->s.eosSlot), slots.data(),
                               sizeof(EosSlot) * nb, hipMemcpyHostToDevice));
@@ -409,7 +410,10 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    const int64_t plane = (int64_t)(align_up(E * cornerBytes) / cornerBytes);
    c->planeStride = plane;
    const int64_t nCorner = sp.nCorner;
-   const unsigned eosBlocks = eos_blocks(sp.numElem);
+   int cus = 0;
+   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
+   c->s.eosShare = eos_share(sp.numElem, cus);
+   const unsigned eosBlocks = eos_blocks(sp.numElem, c->s.eosShare);
 
    // Arena layout.
    struct Slot { void **dst; size_t bytes; };
@@ -481,9 +485,6 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    if (brick) {
       Brick &g = s.brick;
       init_brick(g, sp.sizeX);
-      int cus = 0;
-      if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-         cus = 0;
       int perCu = 0;
       switch (sp.precision) {
       case LGPU_MIXED: perCu = Launch<PolicyMixed>::nodal_brick_blocks_per_cu(); break;
@@ -522,16 +523,17 @@ int set_groups(lgpu_ctx *c, const std::vector<int32_t> &reps, const std::vector<
    regStart[(size_t)numGroups] = (int32_t)at;
    if (at != c->numElem) return LGPU_EINVAL;
    s.numReg = numGroups;
-   const unsigned eosBlocks = eos_blocks(c->numElem);
+   const unsigned eosBlocks = eos_blocks(c->numElem, s.eosShare);
+   const int per = kEosBlock / s.eosShare;
    c->eosBlockRep.assign(eosBlocks, 1);
    for (int i = 0; i < numGroups; ++i)
-      for (int64_t p = regStart[(size_t)i]; p < regStart[(size_t)i + 1]; p += kEosBlock) {
-         const size_t b = (size_t)(p / kEosBlock);
+      for (int64_t p = regStart[(size_t)i]; p < regStart[(size_t)i + 1]; p += per) {
+         const size_t b = (size_t)(p / per);
          c->eosBlockRep[b] = std::max(c->eosBlockRep[b], regRep[(size_t)i]);
       }
    for (int i = 0; i < numGroups; ++i)
       if (regStart[(size_t)i + 1] > regStart[(size_t)i]) {
-         const size_t b = (size_t)((regStart[(size_t)i + 1] - 1) / kEosBlock);
+         const size_t b = (size_t)((regStart[(size_t)i + 1] - 1) / per);
          c->eosBlockRep[b] = std::max(c->eosBlockRep[b], regRep[(size_t)i]);
       }
    c->hostRegStart = regStart;

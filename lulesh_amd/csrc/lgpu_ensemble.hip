@@ -462,6 +462,16 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
       }
    }
    // Offsets.
+   DevState &s = e->s;
+   {
+      int64_t totE = 0;
+      for (int32_t m = 0; m < nMembers; ++m) totE += members[m].numElem;
+      int dev = 0, cus = 0;
+      if (hipGetDevice(&dev) != hipSuccess ||
+          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+         cus = 0;
+      s.eosShare = eos_share(totE, cus);
+   }
    e->nodeStart.assign((size_t)nMembers + 1, 0);
    e->elemStart.assign((size_t)nMembers + 1, 0);
    std::vector<int64_t> cornerStart((size_t)nMembers + 1, 0);
@@ -472,13 +482,13 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
       e->nodeStart[m + 1] = e->nodeStart[m] + d.numNode;
       e->elemStart[m + 1] = e->elemStart[m] + d.numElem;
       cornerStart[m + 1] = cornerStart[m] + d.nodeElemStart[d.numNode];
-      blockStart[m + 1] = blockStart[m] + (int32_t)eos_blocks(d.numElem);
+      blockStart[m + 1] = blockStart[m] + (int32_t)eos_blocks(d.numElem, s.eosShare);
       e->nodeCount.push_back(d.numNode);
       e->elemCount.push_back(d.numElem);
       numRegTot += d.numReg;
    }
    const size_t E = (size_t)e->elemStart[nMembers], N = (size_t)e->nodeStart[nMembers];
-   const size_t nPerm = (size_t)blockStart[nMembers] * kEosBlock;
+   const size_t nPerm = (size_t)blockStart[nMembers] * (kEosBlock / s.eosShare);
    const size_t nCorner = (size_t)cornerStart[nMembers];
    const size_t cb = prec == LGPU_MIXED ? 4 : 8, gb = cb;
    const int64_t plane = (int64_t)(align_up(E * cb) / cb);
@@ -487,7 +497,6 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    // Arena: state first (snapshot-able), then connectivity and scratch.
    struct Slot { void **dst; size_t bytes; };
    std::vector<Slot> slots;
-   DevState &s = e->s;
    auto add = [&](void **dst, size_t bytes) { slots.push_back({dst, align_up(bytes)}); };
    double **stateNode[] = {&s.x, &s.y, &s.z, &s.xd, &s.yd, &s.zd};
    // two doubles of padding, which the kinematics kernel's pair copies may
@@ -585,7 +594,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
       const int32_t ns[3] = {d.numSymmX, d.numSymmY, d.numSymmZ};
       for (int a = 0; a < 3; ++a)
          for (int32_t i = 0; i < ns[a]; ++i) bc[(size_t)(n0 + sy[a][i])] |= (uint8_t)(1u << a);
-      int64_t pos = (int64_t)blockStart[m] * kEosBlock;
+      int64_t pos = (int64_t)blockStart[m] * (kEosBlock / s.eosShare);
       // As for a single domain: the member's elements grouped by EOS repeat
       // count, largest first, in mesh order within a group; the member's
       // remaining region slots stay empty at its end.
@@ -611,7 +620,8 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    // k_eos dispatch slots: blocks in order, each with its repeat counts
    std::vector<int32_t> blockOrder((size_t)blockStart[nMembers]);
    for (size_t b = 0; b < blockOrder.size(); ++b) blockOrder[b] = (int32_t)b;
-   const std::vector<EosSlot> eosSlots = eos_slots(blockOrder, regStart, regRep, (int64_t)nPerm);
+   const std::vector<EosSlot> eosSlots = eos_slots(blockOrder, regStart, regRep, (int64_t)nPerm,
+                                                  s.eosShare);
 
    auto h2d = [&](void *dst, const void *src, size_t bytes) {
       return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess;

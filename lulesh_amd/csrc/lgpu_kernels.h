@@ -232,6 +232,7 @@ struct DevState {
    // count rep0 and the others rep1 (rep0 < 0: look each position up in
    // regStart).  Null (ensembles): block i, counts looked up.
    const struct EosSlot *eosSlot;
+   int32_t eosShare; // k_eos: threads that share an element's repeats
    // Ensemble of independent problems (nMembers > 0): members are
    // concatenated; each has its own dt, loop flag and error flags.
    int32_t nMembers;

@@ -18,9 +18,25 @@ constexpr int kEosBlock = 256;
 // power of two
 constexpr int kDtSlots = 256;
 
-inline unsigned eos_blocks(int numElem)
+// Threads that share an element's repeats in small k_eos launches.
+constexpr int kEosShare = 4;
+
+// Threads per element of k_eos over numElem elements in all: kEosShare up to
+// two waves per SIMD at one thread each (131,072 elements on 256 CUs).
+// Measured, one thread / kEosShare: s=8 13.0 / 7.6 us, s=30 13.9 / 10.6, s=45
+// 15.4 / 13.7, 24 mixed members of 5..24 17.2 / 12.3; above the line s=63
+// mixed (50 repeats) 26.0 / 28.5, s=64 21.3 / 27.3, s=101 49.5 / 67.  Two
+// threads: s=30 10.9, s=64 24.6; eight: s=30 10.4, s=45 17.9.
+inline int eos_share(int64_t numElem, int cus)
 {
-   return (unsigned)((numElem + kEosBlock - 1) / kEosBlock);
+   return numElem <= (int64_t)cus * 4 * 64 * 2 ? kEosShare : 1;
+}
+
+// Workgroups of k_eos over numElem list positions.
+inline unsigned eos_blocks(int numElem, int share)
+{
+   const int per = kEosBlock / share;
+   return (unsigned)((numElem + per - 1) / per);
 }
 
 // k_eos dispatch slots for the perm blocks in `order`: each block's repeat
@@ -30,9 +46,10 @@ inline unsigned eos_blocks(int numElem)
 // block over three or more groups gets rep0 = -1 (k_eos searches regStart).
 inline std::vector<EosSlot> eos_slots(const std::vector<int32_t> &order,
                                       const std::vector<int32_t> &regStart,
-                                      const std::vector<int32_t> &regRep, int64_t numPositions)
+                                      const std::vector<int32_t> &regRep, int64_t numPositions,
+                                      int share)
 {
-   const int ng = (int)regRep.size();
+   const int ng = (int)regRep.size(), per = kEosBlock / share;
    auto group_of = [&](int64_t p) {
       const int g = (int)(std::upper_bound(regStart.begin(), regStart.begin() + ng, (int32_t)p) -
                           regStart.begin()) - 1;
@@ -43,14 +60,14 @@ inline std::vector<EosSlot> eos_slots(const std::vector<int32_t> &order,
    };
    std::vector<EosSlot> slots(order.size());
    for (size_t i = 0; i < order.size(); ++i) {
-      const int64_t p0 = (int64_t)order[i] * kEosBlock;
-      const int64_t p1 = std::max(p0, std::min<int64_t>(p0 + kEosBlock, numPositions) - 1);
+      const int64_t p0 = (int64_t)order[i] * per;
+      const int64_t p1 = std::max(p0, std::min<int64_t>(p0 + per, numPositions) - 1);
       EosSlot &sl = slots[i];
       sl.block = order[i];
       const int g0 = group_of(p0), g1 = group_of(p1);
       if (g0 == g1) {
          sl.rep0 = sl.rep1 = regRep[(size_t)g0];
-         sl.split = (int32_t)(p0 + kEosBlock);
+         sl.split = (int32_t)(p0 + per);
       } else if (group_of(regStart[(size_t)g0 + 1]) == g1) {
          sl.rep0 = regRep[(size_t)g0];
          sl.rep1 = regRep[(size_t)g1];

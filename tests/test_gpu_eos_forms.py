@@ -45,3 +45,27 @@ def test_waves_between_the_volume_limits(precision, eosvmin, eosvmax):
         assert max_rel(fast[f], general[f]) <= TOLERANCE[precision], f
     assert abs(c0 - c1) <= TOLERANCE[precision] * abs(c1)
     assert h0 == h1
+
+
+@pytest.mark.parametrize("s,regions,cost", [(1, 1, 0), (2, 11, 1), (5, 21, 4), (17, 11, 0), (50, 21, 2), (51, 21, 2)])
+def test_elements_phase_with_shared_and_single_threads(s, regions, cost):
+    """Up to 131,072 elements (s <= 50 here) four threads share an element's
+    repeats, above that one thread runs them all: the FP64 elements phase is
+    the oracle's bit for bit on both sides of the line, on partly filled
+    workgroups and with repeat counts below, at and above the thread count."""
+    o = OracleDomain(s, regions, 2, cost)
+    for _ in range(3):
+        o.call("time_increment")
+        assert o.call("lagrange_leapfrog") == 0
+    o.call("time_increment")
+    assert o.call("lagrange_nodal") == 0
+    ctx = context_from_oracle(o)
+    upload_state(ctx, o)
+    assert ctx.lagrange_elements(o.get("deltatime")) == 0
+    status, courant, hydro = ctx.time_constraints()
+    assert status == 0
+    assert o.call("lagrange_elements") == 0
+    o.call("calc_time_constraints")
+    for f in FIELDS:
+        assert np.array_equal(ctx.download(f), o.real(f)), f
+    assert (courant, hydro) == (o.get("dtcourant"), o.get("dthydro"))
