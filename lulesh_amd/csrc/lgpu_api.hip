@@ -492,7 +492,14 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
       default: perCu = Launch<PolicyFp64>::nodal_brick_blocks_per_cu(); break;
       }
       c->brickPerCu = perCu;
-      set_brick_chunk(g, pick_brick_chunk(g, cus * perCu));
+      const int slots = cus * perCu; // k_nodal_block has the walk's occupancy
+      set_brick_chunk(g, pick_brick_chunk(g, slots, 1));
+      s.nodalBlock = slots > 0 && block_is_faster(block_blocks(g), slots,
+                                                  walk_cost((int64_t)g.tilesX * g.tilesY, g.en,
+                                                            slots, g.chunkZ));
+      // the chunk the walk would start from, should an option select it
+      if (s.nodalBlock) set_brick_chunk(g, pick_brick_chunk(g, slots, 4));
+      s.kinFlat = g.s <= kKinFlatMax;
       int kinPerCu = 0;
       switch (sp.precision) {
       case LGPU_MIXED: kinPerCu = Launch<PolicyMixed>::kin_brick_blocks_per_cu(); break;
@@ -1020,6 +1027,7 @@ int lgpu_set_option(lgpu_ctx *c, int option, int64_t value)
    case LGPU_OPT_BRICK_CHUNK:
       if (!c->s.isBrick || value < 1) return LGPU_EINVAL;
       set_brick_chunk(c->s.brick, (int)std::min<int64_t>(value, 1 << 20));
+      c->s.nodalBlock = 0;
       return LGPU_OK;
    case LGPU_OPT_XCD_REMAP:
       c->s.xcdRemap = value ? 1 : 0;
@@ -1027,10 +1035,12 @@ int lgpu_set_option(lgpu_ctx *c, int option, int64_t value)
    case LGPU_OPT_KIN_CHUNK:
       if (!c->s.isBrick || value < 1) return LGPU_EINVAL;
       set_kin_chunk(c->s.brick, (int)std::min<int64_t>(value, 1 << 20));
+      c->s.kinFlat = 0;
       return LGPU_OK;
    case LGPU_OPT_BRICK_ROWS:
       if (!c->s.isBrick || (value != 8 && value != 16)) return LGPU_EINVAL;
       set_brick_tile(c->s.brick, 16, (int)value);
+      c->s.nodalBlock = 0;
       return LGPU_OK;
    case LGPU_OPT_EOS_INTERLEAVE:
       if (value < 0 || value > 1024) return LGPU_EINVAL;

@@ -92,20 +92,24 @@ inline void set_brick_chunk(Brick &g, int chunk)
    g.chunks = (g.en + g.chunkZ - 1) / g.chunkZ;
 }
 
-// Planes per workgroup of a column-walking kernel: a launch of `columns`
-// column tiles, each cut into z-chunks of `chunk` planes out of `planes`,
-// runs in rounds of `slots` resident workgroups, and a workgroup walks one
-// plane more than its chunk.  Picks the chunk that minimises rounds x
-// (chunk + 1): redundant planes against a partly filled last round.
-inline int pick_chunk(int64_t columns, int planes, int slots, int fallback)
+// Time of a column-walking launch in planes: `columns` column tiles, each cut
+// into z-chunks of `chunk` planes out of `planes`, run in rounds of `slots`
+// resident workgroups, and a workgroup walks one plane more than its chunk.
+inline int64_t walk_cost(int64_t columns, int planes, int slots, int chunk)
+{
+   const int64_t blocks = columns * ((planes + chunk - 1) / chunk);
+   return (blocks + slots - 1) / slots * (chunk + 1);
+}
+
+// The chunk (at least `least` planes) with the smallest walk_cost: redundant
+// planes against a partly filled last round.
+inline int pick_chunk(int64_t columns, int planes, int slots, int least, int fallback)
 {
    if (slots < 1) return fallback;
    int best = fallback;
-   double bestCost = 1e300;
-   for (int ch = 4; ch <= planes; ++ch) {
-      const int64_t blocks = columns * ((planes + ch - 1) / ch);
-      const int64_t rounds = (blocks + slots - 1) / slots;
-      const double cost = (double)rounds * (ch + 1);
+   int64_t bestCost = INT64_MAX;
+   for (int ch = least; ch <= planes; ++ch) {
+      const int64_t cost = walk_cost(columns, planes, slots, ch);
       if (cost < bestCost) {
          bestCost = cost;
          best = ch;
@@ -117,9 +121,9 @@ inline int pick_chunk(int64_t columns, int planes, int slots, int fallback)
 // Default node planes per workgroup of the fused nodal kernel.  s=192 on
 // 256 CUs: 65 for FP64 (2 workgroups per CU: all 507 resident at once, 2%
 // faster than 22), 22 for the mixed form (3 per CU).
-inline int pick_brick_chunk(const Brick &g, int slots)
+inline int pick_brick_chunk(const Brick &g, int slots, int least)
 {
-   return pick_chunk((int64_t)g.tilesX * g.tilesY, g.en, slots, 8);
+   return pick_chunk((int64_t)g.tilesX * g.tilesY, g.en, slots, least, 8);
 }
 
 inline void set_kin_chunk(Brick &g, int chunk)
@@ -133,7 +137,7 @@ inline void set_kin_chunk(Brick &g, int chunk)
 // CU: 1,008 workgroups, all resident at once; 3% faster than 12).
 inline int pick_kin_chunk(const Brick &g, int slots)
 {
-   return pick_chunk((int64_t)g.kinTiles * g.kinTiles, g.s, slots, 12);
+   return pick_chunk((int64_t)g.kinTiles * g.kinTiles, g.s, slots, 4, 12);
 }
 
 // Fused nodal kernel tiles of w threads by h rows: (w-1) x (h-1) nodes each.
@@ -200,6 +204,55 @@ inline void pick_member_kin_tile(Brick &g)
    set_kin_tile(g, bestW, 256 / bestW);
 }
 
+// k_nodal_block: the block of at most 256 elements that covers the nodes with
+// the fewest workgroups; ties go to the widest (rows of 16-byte loads).
+inline void pick_nodal_block(Brick &g)
+{
+   auto tiles = [&](int n) { return (g.en + n - 2) / (n - 1); };
+   int64_t best = INT64_MAX;
+   for (int w = 3; w <= 18; ++w)
+      for (int h = 3; w * h * 3 <= 256; ++h) {
+         const int d = 256 / (w * h);
+         const int64_t n = (int64_t)tiles(w) * tiles(h) * tiles(d);
+         if (n <= best) {
+            best = n;
+            g.blkW = w;
+            g.blkH = h;
+            g.blkD = d;
+         }
+      }
+   g.blkX = tiles(g.blkW);
+   g.blkY = tiles(g.blkH);
+   g.blkZ = tiles(g.blkD);
+}
+
+inline int64_t block_blocks(const Brick &g) { return (int64_t)g.blkX * g.blkY * g.blkZ; }
+
+// True when k_nodal_block is the faster nodal kernel: `blocks` workgroups of
+// it on `slots` resident ones take about 1 + blocks / slots planes of the
+// walking kernel's time (8.3 us a plane in FP64: s=30 11.1, s=45 21.1, s=64
+// 38.5, s=74 55.1 us), and the walk its `cost` and, with its start and end,
+// 0.4 more.  Block / walk, FP64: s=8 10.6 / 14.9 us, s=30 11.1 / 25.9, s=45
+// 21.1 / 41.5, s=60 34.4 / 41.4, s=76 53.8 / 55.7; walk taken: s=59 31.5 /
+// 27.8, s=74 55.1 / 42.5, s=101 119.8 / 92.3.  FP64_FMA s=64 33.9 / 35.0,
+// mixed s=30 9.8 / 13.7, s=63 25.0 / 26.7.
+inline bool block_is_faster(int64_t blocks, int slots, int64_t cost)
+{
+   return slots > 0 && 5 * blocks < (5 * cost - 3) * slots;
+}
+
+// The largest brick of k_kin_flat.  Flat / best walk: FP64 s=30 8.5 / 9.0 us
+// (14.9 at the walk's own choice), s=64 14.3 / 16.0, s=101 34.2 / 43.2, s=115
+// 56.0 / 61.3, s=118 62.0 / 62.2, s=120 64.2 / 63.4, s=128 76.3 / 66.0, s=192
+// 248 / 198; mixed s=105 26.3 / 30.6, s=115 41.5 / 44.1, s=120 50.5 / 47.1.
+// Above it the elements in flight on an XCD, and the planes they read, no
+// longer stay in its L2.  Ensembles: each member's own size counts (64 of
+// 16..64, 6.0 M elements: FP64 179.5 / 203, mixed 140 / 146).
+constexpr int kKinFlatMax = 117; // elements per edge
+
+// Workgroups of k_kin_flat: 256 elements each.
+inline int64_t flat_blocks(const Brick &g) { return ((int64_t)g.s * g.s * g.s + 255) / 256; }
+
 // Tiling of an s^3 brick with the default chunks (the caller may pick
 // others): 15x15-node tiles of the fused nodal kernel, 16x16-element tiles
 // of the kinematics kernel.
@@ -214,6 +267,7 @@ inline void init_brick(Brick &g, int s)
    set_kin_tile(g, 16, 16);
    set_brick_chunk(g, 8);
    set_kin_chunk(g, 12);
+   pick_nodal_block(g);
 }
 
 // Workgroups of one launch of each brick kernel.

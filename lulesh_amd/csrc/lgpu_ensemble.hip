@@ -289,7 +289,57 @@ int launch_graph(lgpu_ensemble *e)
    return LGPU_OK;
 }
 
-// Member tables of the brick path for the current chunk choices: per-member
+// The brick path's default kernels and nodal chunk.  A walk's cost is taken
+// over all members' workgroups; within it the chunk with the least work per
+// resident workgroup, plus half a walk for the tail of the launch (the
+// members' last chunks are shorter, so rounds do not end together).  64
+// members of 16..64, FP64: chunk 10, 500 us (7: 495, 4: 519); 30 of 10..40:
+// chunk 4, 68.7 us (8: 81.8, k_nodal_block 84.8); 24 of 5..24: k_nodal_block,
+// FP64 18.6 and mixed 13.6 us (best walk 24.1 and 18.5).
+void pick_brick_kernels(lgpu_ensemble *e)
+{
+   int dev = 0, cus = 0, perCu = 0, largest = 0;
+   if (hipGetDevice(&dev) != hipSuccess ||
+       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      cus = 0;
+   switch (e->precision) {
+   case LGPU_MIXED: perCu = Launch<PolicyMixed>::nodal_brick_blocks_per_cu(); break;
+   case LGPU_FP64_FMA: perCu = Launch<PolicyFp64Fma>::nodal_brick_blocks_per_cu(); break;
+   default: perCu = Launch<PolicyFp64>::nodal_brick_blocks_per_cu(); break;
+   }
+   const int slots = cus * perCu;
+   std::vector<Brick> bricks;
+   int64_t blocks = 0;
+   for (int32_t sz : e->memberSize) {
+      Brick g{};
+      init_brick(g, sz);
+      pick_member_tile(g);
+      blocks += block_blocks(g);
+      largest = std::max(largest, sz);
+      bricks.push_back(g);
+   }
+   e->s.kinFlat = largest <= kKinFlatMax;
+   if (slots < 1) return;
+   int64_t least = INT64_MAX;
+   double best = 1e300;
+   for (int ch = 1; ch <= 22; ++ch) {
+      int64_t walks = 0, planes = 0;
+      for (const Brick &g : bricks) {
+         const int64_t chunks = (g.en + ch - 1) / ch;
+         walks += (int64_t)g.tilesX * g.tilesY * chunks;
+         planes += (int64_t)g.tilesX * g.tilesY * (g.en + chunks);
+      }
+      least = std::min(least, (walks + slots - 1) / slots * (ch + 1));
+      const double work = std::max((double)planes / slots + 0.5 * (ch + 1), ch + 1.0);
+      if (work < best) {
+         best = work;
+         e->nodalChunk = ch;
+      }
+   }
+   e->s.nodalBlock = block_is_faster(blocks, slots, least);
+}
+
+// Member tables of the brick path for the current kernel and chunk choices: per-member
 // bricks with offsets and first workgroups, and workgroup -> member maps.
 int build_brick_tables(lgpu_ensemble *e)
 {
@@ -309,7 +359,8 @@ int build_brick_tables(lgpu_ensemble *e)
       mb[(size_t)m].elemOff = e->elemStart[(size_t)m];
       mb[(size_t)m].nodalBlock0 = (int32_t)nb;
       mb[(size_t)m].kinBlock0 = (int32_t)kb;
-      const int64_t n1 = nodal_blocks(g), k1 = kin_blocks(g);
+      const int64_t n1 = e->s.nodalBlock ? block_blocks(g) : nodal_blocks(g);
+      const int64_t k1 = e->s.kinFlat ? flat_blocks(g) : kin_blocks(g);
       nodalOf.insert(nodalOf.end(), (size_t)n1, m);
       kinOf.insert(kinOf.end(), (size_t)k1, m);
       nb += n1;
@@ -645,6 +696,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
              h2d((void *)s.memberBlockStart, blockStart.data(), 4 * blockStart.size()) &&
              h2d(s.v, ones.data(), 8 * E);
    if (!ok) return bail(LGPU_EDEVICE);
+   if (e->brick) pick_brick_kernels(e);
    if (e->brick && build_brick_tables(e) != LGPU_OK) return bail(LGPU_EDEVICE);
    if (hipHostMalloc((void **)&e->host, (size_t)nMembers * (9 * 8 + 8) + 64 +
                                             (size_t)nMembers * kNumErrSites * 4,
@@ -832,7 +884,14 @@ int lgpu_ensemble_set_option(lgpu_ensemble *e, int option, int64_t value)
    case LGPU_ENS_OPT_BRICK_CHUNK:
    case LGPU_ENS_OPT_KIN_CHUNK:
       if (!e->brick || value < 1 || value > 1024) return LGPU_EINVAL;
-      (option == LGPU_ENS_OPT_BRICK_CHUNK ? e->nodalChunk : e->kinChunk) = (int)value;
+      // a chunk asks for the kernel that walks up columns
+      if (option == LGPU_ENS_OPT_BRICK_CHUNK) {
+         e->nodalChunk = (int)value;
+         e->s.nodalBlock = 0;
+      } else {
+         e->kinChunk = (int)value;
+         e->s.kinFlat = 0;
+      }
       return build_brick_tables(e);
    default:
       return LGPU_EINVAL;
@@ -894,12 +953,21 @@ int lgpu_ensemble_autotune(lgpu_ensemble *e, const lgpu_time_state *ts, int32_t 
    };
    int r = LGPU_OK;
    if (e->brick) {
-      // Chunk of each fused kernel over a few candidates, then the XCD mapping.
-      const int nodalCands[] = {4, 6, 8, 11, 16, 22}, kinCands[] = {4, 6, 8, 12, 16};
+      // k_nodal_block and k_kin_flat (candidate 0) and the chunks of the
+      // walking kernels, then the XCD mapping.
+      const int nodalCands[] = {0, 2, 4, 6, 8, 11, 16, 22}, kinCands[] = {0, 4, 6, 8, 12, 16};
       float best = 1e30f;
       int bestC = e->nodalChunk;
+      auto set_nodal = [&](int c) {
+         e->s.nodalBlock = c == 0;
+         if (c) e->nodalChunk = c;
+      };
+      auto set_kin = [&](int c) {
+         e->s.kinFlat = c == 0;
+         if (c) e->kinChunk = c;
+      };
       for (int c : nodalCands) {
-         e->nodalChunk = c;
+         set_nodal(c);
          r = build_brick_tables(e);
          float ms[kENumKernels];
          if (!r) r = trial(ms);
@@ -909,12 +977,12 @@ int lgpu_ensemble_autotune(lgpu_ensemble *e, const lgpu_time_state *ts, int32_t 
             bestC = c;
          }
       }
-      e->nodalChunk = bestC;
+      set_nodal(bestC);
       best = 1e30f;
       bestC = e->kinChunk;
       for (int c : kinCands) {
          if (r) break;
-         e->kinChunk = c;
+         set_kin(c);
          r = build_brick_tables(e);
          float ms[kENumKernels];
          if (!r) r = trial(ms);
@@ -924,7 +992,7 @@ int lgpu_ensemble_autotune(lgpu_ensemble *e, const lgpu_time_state *ts, int32_t 
             bestC = c;
          }
       }
-      e->kinChunk = bestC;
+      set_kin(bestC);
       if (!r) r = build_brick_tables(e);
    } else {
       // Each of the three launch-shape-sensitive kernels is tuned over the

@@ -109,6 +109,8 @@ struct PolicyFp64 {
    // 476.5 us (device loop: FP64 unchanged, FP64_FMA 484 -> 472 us); mixed
    // 417.5 -> 420.4 us
    static constexpr bool kNodePhasePrio = true;
+   // k_nodal_block waves per SIMD
+   static constexpr int kBlockWaves = 2;
 };
 
 // The FP64 policy compiled with multiply-add contraction (its own
@@ -138,6 +140,7 @@ struct PolicyMixed {
    // k_eos at 8 waves per SIMD (at most 64 VGPRs): 214 -> 211 us at s=192
    static constexpr int kEosWaves = 8;
    static constexpr bool kNodePhasePrio = false;
+   static constexpr int kBlockWaves = 3;
 };
 
 // Element i of a device array through a 32-bit byte offset: the access
@@ -175,6 +178,9 @@ struct Brick {
    int32_t kinTiles, kinChunk, kinChunks;
    // ensemble members: kinW x kinH element tiles, kinTilesX x kinTilesY per plane
    int32_t kinW, kinH, kinTilesX, kinTilesY;
+   // k_nodal_block: blkW x blkH x blkD elements per workgroup, blkX x blkY x
+   // blkZ workgroups
+   int32_t blkW, blkH, blkD, blkX, blkY, blkZ;
 };
 
 // One ensemble member on the brick path: its brick, where its nodes and
@@ -226,6 +232,8 @@ struct DevState {
    struct DevTime *time;
    Brick brick;             // valid when isBrick
    int32_t isBrick;
+   int32_t nodalBlock; // nodal pass by k_nodal_block instead of k_nodal_brick
+   int32_t kinFlat;    // kinematics by k_kin_flat instead of k_kin_brick
    int32_t brickFaces; // k_eos computes face neighbours and BC masks from the brick
    // k_eos dispatch table (one problem): workgroup i processes perm block
    // eosSlot[i].block, whose positions below eosSlot[i].split take repeat
