@@ -38,6 +38,12 @@ constexpr size_t kAlign = 256;
 
 inline size_t align_up(size_t v) { return (v + kAlign - 1) & ~(kAlign - 1); }
 
+// A k_eos slot and its first element.
+struct PlacedSlot {
+   EosSlot slot;
+   int32_t elem;
+};
+
 struct TimedLaunch {
    int kernel;
    hipEvent_t start, stop;
@@ -52,8 +58,7 @@ struct lgpu_ctx {
    int32_t sizeX = 0;
    int block = 256;
    bool keepDiag = false;
-   std::vector<int32_t> eosBlockRep; // repeat count of each k_eos block (region order)
-   std::vector<int32_t> hostRegStart, hostRegRep; // the work-list groups (host copies)
+   std::vector<PlacedSlot> eosSlots; // in work-list order
    int eosInterleave = 0;
    int32_t brickPerCu = 0;
    bool timing = false;
@@ -195,53 +200,49 @@ int validate(const lgpu_mesh_desc *d, std::string &why)
    return LGPU_OK;
 }
 
-// EOS repeat count of region r, lulesh.cc:2390-2400.
-int32_t region_rep(int32_t r, int32_t numReg, int32_t cost)
-{
-   if (r < numReg / 2) return 1;
-   if (r < numReg - (numReg + 15) / 20) return 1 + cost;
-   return 10 * (1 + cost);
-}
-
 // k_eos dispatch order.  k = 0: work-list order (largest repeat count
 // first).  k > 0: the workgroups of the largest repeat count are spread out,
-// one every k + 1 dispatches, with the others (in list order) between them,
-// so that compute-bound and memory-bound workgroups share the CUs.  The
+// one every k + 1 dispatches, with the others between them, so that
+// compute-bound and memory-bound workgroups share the CUs.  The others come in
+// the order of their place in the mesh, whatever their repeat count, so that
+// the neighbour gradients and partly used lines of one part of the mesh are
+// fetched while they are in the caches (s=192, k = 4: FP64 r21 299.6 -> 291.3
+// us, mixed r11 207 -> 190.8 us against one repeat count after the other; the
+// heavy workgroups in mesh order too: 302-323 and 193-203 us).  The
 // dispatcher deals workgroups to the 8 XCDs in turn, so an even period would
 // put every heavy workgroup on the same few XCDs (measured: period 4 nearly
 // doubles the EOS time); an even k + 1 is raised to the next odd period.
 int set_eos_order(lgpu_ctx *c, int k)
 {
    if (k > 0 && (k + 1) % 2 == 0) ++k;
-   const size_t nb = c->eosBlockRep.size();
-   std::vector<int32_t> order;
-   order.reserve(nb);
+   std::vector<EosSlot> slots;
    if (k <= 0) {
-      for (size_t b = 0; b < nb; ++b) order.push_back((int32_t)b);
+      for (const PlacedSlot &p : c->eosSlots) slots.push_back(p.slot);
    } else {
-      const int32_t top = *std::max_element(c->eosBlockRep.begin(), c->eosBlockRep.end());
-      std::vector<int32_t> heavy, rest;
-      for (size_t b = 0; b < nb; ++b) (c->eosBlockRep[b] == top ? heavy : rest).push_back((int32_t)b);
-      // The FP64 forms walk each group from the top of the mesh down: the
-      // kinematics pass before k_eos sweeps the mesh bottom to top, so its
-      // last outputs are still in the caches when k_eos starts (s=192, 21
-      // regions: k_eos 367 -> 357 us; the mixed form gains nothing and its
-      // next nodal pass loses 2 us, so it keeps the ascending walk).
+      std::vector<PlacedSlot> heavy, rest;
+      for (const PlacedSlot &p : c->eosSlots)
+         (p.slot.rep == c->eosSlots.front().slot.rep ? heavy : rest).push_back(p);
+      std::stable_sort(rest.begin(), rest.end(),
+                       [](const PlacedSlot &a, const PlacedSlot &b) { return a.elem < b.elem; });
+      // The FP64 forms walk the mesh from the top down: the kinematics pass
+      // before k_eos sweeps it bottom to top, so its last outputs are still
+      // in the caches when k_eos starts (s=192, 21 regions: k_eos 367 -> 357
+      // us; the mixed form gains nothing and its next nodal pass loses 2 us,
+      // so it keeps the ascending walk).
       if (c->precision != LGPU_MIXED) {
          std::reverse(heavy.begin(), heavy.end());
          std::reverse(rest.begin(), rest.end());
       }
       size_t h = 0, r = 0;
       while (h < heavy.size() || r < rest.size()) {
-         if (h < heavy.size()) order.push_back(heavy[h++]);
-         for (int j = 0; j < k && r < rest.size(); ++j) order.push_back(rest[r++]);
+         if (h < heavy.size()) slots.push_back(heavy[h++].slot);
+         for (int j = 0; j < k && r < rest.size(); ++j) slots.push_back(rest[r++].slot);
       }
    }
-   const std::vector<EosSlot> slots = eos_slots(order, c->hostRegStart, c->hostRegRep, c->numElem,
-                                               c->s.eosShare);
+   c->s.eosBlocks = (int32_t)slots.size();
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
    HIP_OR_RETURN(c, hipMemcpy(const_cast<EosSlot *>(c->s.eosSlot), slots.data(),
-                              sizeof(EosSlot) * nb, hipMemcpyHostToDevice));
+                              sizeof(EosSlot) * slots.size(), hipMemcpyHostToDevice));
    c->eosInterleave = std::max(0, k);
    return LGPU_OK;
 }
@@ -412,8 +413,9 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    const int64_t nCorner = sp.nCorner;
    int cus = 0;
    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
-   c->s.eosShare = eos_share(sp.numElem, cus);
-   const unsigned eosBlocks = eos_blocks(sp.numElem, c->s.eosShare);
+   c->s.eosSplit = eos_split(sp.numElem) ? 1 : 0;
+   // every group may end in a partly filled workgroup
+   const size_t eosBlocks = E / (size_t)(kEosBlock / (c->s.eosSplit ? kEosShare : 1)) + 4;
 
    // Arena layout.
    struct Slot { void **dst; size_t bytes; };
@@ -443,8 +445,6 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    if (!brick) add(&s.corner, cornerBytes * (size_t)plane * 48);
    add((void **)&s.perm, sizeof(int32_t) * E);
    add((void **)&s.eosSlot, sizeof(EosSlot) * eosBlocks);
-   add((void **)&s.regStart, sizeof(int32_t) * (size_t)(sp.numReg + 1));
-   add((void **)&s.regRep, sizeof(int32_t) * (size_t)sp.numReg);
    add((void **)&s.err, sizeof(int32_t) * kNumErrSites);
    add((void **)&s.dtPartial, sizeof(double) * 2 * kDtSlots);
    add((void **)&s.dtOut, sizeof(double) * 2);
@@ -477,8 +477,6 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    }
    s.numElem = sp.numElem;
    s.numNode = sp.numNode;
-   s.numReg = sp.numReg;
-   s.numPerm = sp.numElem;
    s.xcdRemap = 1;
    s.isBrick = brick ? 1 : 0;
    s.brickFaces = (brick && sp.brickFaces) ? 1 : 0;
@@ -512,44 +510,37 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    return LGPU_OK;
 }
 
-// The EOS work-list groups: one per distinct repeat count, largest first,
-// with their sizes; the elements of group i are perm[regStart[i] ..
-// regStart[i+1]).  Uploads regStart/regRep and derives the repeat count of
-// each k_eos block (the largest over the groups it holds).
-int set_groups(lgpu_ctx *c, const std::vector<int32_t> &reps, const std::vector<int64_t> &sizes)
-{
-   DevState &s = c->s;
-   const int numGroups = std::max<int>(1, (int)reps.size());
-   std::vector<int32_t> regStart((size_t)numGroups + 1, 0), regRep((size_t)numGroups, 1);
-   int64_t at = 0;
-   for (size_t k = 0; k < reps.size(); ++k) {
-      regStart[k] = (int32_t)at;
-      regRep[k] = reps[k];
-      at += sizes[k];
+// The EOS work list's slots, from its groups (one per distinct repeat count,
+// largest first, in the order of perm).  The list of a group is made of runs
+// of consecutive elements, run i being elements runElem[i].. at positions
+// runPos[i].. up to runPos[i + 1] of it.
+struct EosRuns {
+   std::vector<int64_t> pos;
+   std::vector<int32_t> elem;
+   void add(int64_t at, int32_t first)
+   {
+      pos.push_back(at);
+      elem.push_back(first);
    }
-   regStart[(size_t)numGroups] = (int32_t)at;
-   if (at != c->numElem) return LGPU_EINVAL;
-   s.numReg = numGroups;
-   const unsigned eosBlocks = eos_blocks(c->numElem, s.eosShare);
-   const int per = kEosBlock / s.eosShare;
-   c->eosBlockRep.assign(eosBlocks, 1);
-   for (int i = 0; i < numGroups; ++i)
-      for (int64_t p = regStart[(size_t)i]; p < regStart[(size_t)i + 1]; p += per) {
-         const size_t b = (size_t)(p / per);
-         c->eosBlockRep[b] = std::max(c->eosBlockRep[b], regRep[(size_t)i]);
+};
+
+int set_groups(lgpu_ctx *c, const std::vector<int32_t> &reps, const std::vector<EosRuns> &runs,
+               const std::vector<int64_t> &sizes)
+{
+   c->eosSlots.clear();
+   int64_t at = 0;
+   for (size_t g = 0; g < reps.size(); ++g) {
+      std::vector<EosSlot> slots;
+      add_eos_slots(slots, EosGroup{at, sizes[g], reps[g]}, c->s.eosSplit != 0);
+      size_t r = 0;
+      for (const EosSlot &sl : slots) {
+         const int64_t p = sl.pos - at;
+         while (r + 1 < runs[g].pos.size() && runs[g].pos[r + 1] <= p) ++r;
+         c->eosSlots.push_back(PlacedSlot{sl, (int32_t)(runs[g].elem[r] + (p - runs[g].pos[r]))});
       }
-   for (int i = 0; i < numGroups; ++i)
-      if (regStart[(size_t)i + 1] > regStart[(size_t)i]) {
-         const size_t b = (size_t)((regStart[(size_t)i + 1] - 1) / per);
-         c->eosBlockRep[b] = std::max(c->eosBlockRep[b], regRep[(size_t)i]);
-      }
-   c->hostRegStart = regStart;
-   c->hostRegRep = regRep;
-   HIP_OR_RETURN(c, hipMemcpy(const_cast<int32_t *>(s.regStart), regStart.data(),
-                              sizeof(int32_t) * regStart.size(), hipMemcpyHostToDevice));
-   HIP_OR_RETURN(c, hipMemcpy(const_cast<int32_t *>(s.regRep), regRep.data(),
-                              sizeof(int32_t) * regRep.size(), hipMemcpyHostToDevice));
-   return LGPU_OK;
+      at += sizes[g];
+   }
+   return at == c->numElem ? LGPU_OK : LGPU_EINVAL;
 }
 
 // Last steps of both constructors: the EOS dispatch order and the pinned
@@ -665,8 +656,7 @@ int lgpu_create(const lgpu_mesh_desc *d, lgpu_ctx **out)
    // runs the same code for every region), so merging the regions of equal
    // count into one ascending list is exact; it turns the regions' short runs
    // (~38 elements on average) into long ones, so k_eos reads whole cache
-   // lines.  regStart/regRep then describe the groups (k_eos reads a
-   // block's counts from its dispatch slot, built from them).
+   // lines.
    std::vector<int32_t> perm;
    perm.reserve(E);
    std::vector<int32_t> repOf(E, 1);
@@ -679,11 +669,18 @@ int lgpu_create(const lgpu_mesh_desc *d, lgpu_ctx **out)
    }
    std::sort(reps.begin(), reps.end(), std::greater<int32_t>());
    std::vector<int64_t> sizes;
+   std::vector<EosRuns> runs;
    for (int32_t rep : reps) {
       const size_t before = perm.size();
-      for (size_t el = 0; el < E; ++el)
-         if (repOf[el] == rep) perm.push_back((int32_t)el);
+      EosRuns run;
+      for (size_t el = 0; el < E; ++el) {
+         if (repOf[el] != rep) continue;
+         if (perm.size() == before || perm.back() + 1 != (int32_t)el)
+            run.add((int64_t)(perm.size() - before), (int32_t)el);
+         perm.push_back((int32_t)el);
+      }
       sizes.push_back((int64_t)(perm.size() - before));
+      runs.push_back(run);
    }
    std::vector<double> ones(E, 1.0);
 
@@ -701,7 +698,7 @@ int lgpu_create(const lgpu_mesh_desc *d, lgpu_ctx **out)
              h2d(s.perm, perm.data(), sizeof(int32_t) * E) &&
              h2d(s.v, ones.data(), sizeof(double) * E);
    if (!ok) return fail(LGPU_EDEVICE);
-   if ((st = set_groups(c, reps, sizes)) != LGPU_OK) return fail(st);
+   if ((st = set_groups(c, reps, runs, sizes)) != LGPU_OK) return fail(st);
    if ((st = finish_context(c)) != LGPU_OK) return fail(st);
    *out = c;
    return LGPU_OK;
@@ -755,9 +752,12 @@ int lgpu_create_sedov(const lgpu_sedov_desc *d, lgpu_ctx **out, lgpu_time_state 
       if (regSize[(size_t)r] > 0) groupSize[group_of(r + 1)] += regSize[(size_t)r];
    for (size_t g = 1; g < reps.size(); ++g) groupAt[g] = groupAt[g - 1] + groupSize[g - 1];
    std::vector<int32_t> runDest((size_t)d->numRuns);
+   std::vector<EosRuns> runs(reps.size());
+   const std::vector<int64_t> groupStart = groupAt;
    for (int32_t r = 0; r < d->numRuns; ++r) {
       const size_t g = group_of(d->runReg[r]);
       runDest[(size_t)r] = (int32_t)groupAt[g];
+      runs[g].add(groupAt[g] - groupStart[g], runStart[(size_t)r]);
       groupAt[g] += d->runLen[r];
    }
 
@@ -800,7 +800,7 @@ int lgpu_create_sedov(const lgpu_sedov_desc *d, lgpu_ctx **out, lgpu_time_state 
    if (hipStreamSynchronize(c->stream) != hipSuccess) return fail(LGPU_EDEVICE);
    (void)hipFree(runTables);
    runTables = nullptr;
-   if ((st = set_groups(c, reps, groupSize)) != LGPU_OK) return fail(st);
+   if ((st = set_groups(c, reps, runs, groupSize)) != LGPU_OK) return fail(st);
    if ((st = finish_context(c)) != LGPU_OK) return fail(st);
 
    // Energy deposit and first dt (lulesh-init.cc:180-192).

@@ -86,13 +86,6 @@ __global__ void k_time_increment_ens(EnsTime t, const double *dtOut, const int32
    t.cycle[m] += 1;
 }
 
-int32_t region_rep(int32_t r, int32_t numReg, int32_t cost)
-{
-   if (r < numReg / 2) return 1;
-   if (r < numReg - (numReg + 15) / 20) return 1 + cost;
-   return 10 * (1 + cost);
-}
-
 } // namespace
 
 struct lgpu_ensemble {
@@ -489,6 +482,9 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    // kernels are not asked for).
    e->brick = !(members[0].flags & LGPU_FLAG_GENERIC);
    for (int32_t m = 0; m < nMembers && e->brick; ++m) e->brick = is_reference_brick(&members[m]);
+   e->s.brickFaces = e->brick ? 1 : 0;
+   for (int32_t m = 0; m < nMembers && e->s.brickFaces; ++m)
+      e->s.brickFaces = brick_faces_computable(&members[m]) ? 1 : 0;
    for (int32_t m = 0; m < nMembers; ++m) e->memberSize.push_back(members[m].sizeX);
    const lgpu_constants &kk = members[0].k;
    e->k = Consts{kk.e_cut, kk.p_cut, kk.q_cut, kk.v_cut, kk.u_cut, kk.hgcoef, kk.ss4o3,
@@ -517,29 +513,41 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    {
       int64_t totE = 0;
       for (int32_t m = 0; m < nMembers; ++m) totE += members[m].numElem;
-      int dev = 0, cus = 0;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-         cus = 0;
-      s.eosShare = eos_share(totE, cus);
+      s.eosSplit = eos_split(totE) ? 1 : 0;
    }
    e->nodeStart.assign((size_t)nMembers + 1, 0);
    e->elemStart.assign((size_t)nMembers + 1, 0);
    std::vector<int64_t> cornerStart((size_t)nMembers + 1, 0);
-   std::vector<int32_t> blockStart((size_t)nMembers + 1, 0);
-   int64_t numRegTot = 0;
+   // The EOS work list, as for a single domain: each member's elements grouped
+   // by EOS repeat count, largest first, in mesh order within a group.
+   std::vector<int32_t> perm, blockMember, blockStart(1, 0);
+   std::vector<EosSlot> eosSlots;
    for (int32_t m = 0; m < nMembers; ++m) {
       const lgpu_mesh_desc &d = members[m];
       e->nodeStart[m + 1] = e->nodeStart[m] + d.numNode;
       e->elemStart[m + 1] = e->elemStart[m] + d.numElem;
       cornerStart[m + 1] = cornerStart[m] + d.nodeElemStart[d.numNode];
-      blockStart[m + 1] = blockStart[m] + (int32_t)eos_blocks(d.numElem, s.eosShare);
       e->nodeCount.push_back(d.numNode);
       e->elemCount.push_back(d.numElem);
-      numRegTot += d.numReg;
+      const int32_t e0 = e->elemStart[m];
+      std::vector<int32_t> repOf((size_t)d.numElem, 1), reps;
+      for (int32_t r = 0; r < d.numReg; ++r) {
+         const int32_t rep = region_rep(r, d.numReg, d.cost);
+         if (d.regElemSize[r] > 0 && std::find(reps.begin(), reps.end(), rep) == reps.end())
+            reps.push_back(rep);
+         for (int32_t i = 0; i < d.regElemSize[r]; ++i) repOf[(size_t)d.regElemlist[r][i]] = rep;
+      }
+      std::sort(reps.begin(), reps.end(), std::greater<int32_t>());
+      for (int32_t rep : reps) {
+         const int64_t pos = (int64_t)perm.size();
+         for (int32_t el = 0; el < d.numElem; ++el)
+            if (repOf[(size_t)el] == rep) perm.push_back(el + e0);
+         add_eos_slots(eosSlots, EosGroup{pos, (int64_t)perm.size() - pos, rep}, s.eosSplit != 0);
+      }
+      blockMember.resize(eosSlots.size(), m);
+      blockStart.push_back((int32_t)eosSlots.size());
    }
    const size_t E = (size_t)e->elemStart[nMembers], N = (size_t)e->nodeStart[nMembers];
-   const size_t nPerm = (size_t)blockStart[nMembers] * (kEosBlock / s.eosShare);
    const size_t nCorner = (size_t)cornerStart[nMembers];
    const size_t cb = prec == LGPU_MIXED ? 4 : 8, gb = cb;
    const int64_t plane = (int64_t)(align_up(E * cb) / cb);
@@ -584,9 +592,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    const int32_t **nbr[] = {&s.lxim, &s.lxip, &s.letam, &s.letap, &s.lzetam, &s.lzetap, &s.elemBC};
    for (const int32_t **p : nbr) add((void **)p, 4 * E);
    if (!e->brick) add(&s.corner, cb * (size_t)plane * 48);
-   add((void **)&s.perm, 4 * nPerm);
-   add((void **)&s.regStart, 4 * ((size_t)numRegTot + 1));
-   add((void **)&s.regRep, 4 * (size_t)numRegTot);
+   add((void **)&s.perm, 4 * E);
    add((void **)&s.err, 4 * kNumErrSites);
    add((void **)&s.dtPartial, 16 * (size_t)blockStart[nMembers]);
    add((void **)&s.dtOut, 16);
@@ -614,8 +620,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    }
    s.numElem = (int32_t)E;
    s.numNode = (int32_t)N;
-   s.numReg = (int32_t)numRegTot;
-   s.numPerm = (int32_t)nPerm;
+   s.eosBlocks = blockStart[nMembers];
    s.xcdRemap = 1;
    s.isBrick = 0;
    s.nMembers = nMembers;
@@ -623,12 +628,9 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    s.memberActive = t.active;
 
    // Concatenated connectivity.
-   std::vector<int32_t> nodelist(8 * E), nbrs[7], nodeElemStart(N + 1), corner(nCorner), perm(nPerm, -1);
+   std::vector<int32_t> nodelist(8 * E), nbrs[7], nodeElemStart(N + 1), corner(nCorner);
    for (auto &v : nbrs) v.assign(E, 0);
-   std::vector<int32_t> regStart((size_t)numRegTot + 1, 0), regRep((size_t)numRegTot, 1);
-   std::vector<int32_t> blockMember((size_t)blockStart[nMembers], -1);
    std::vector<uint8_t> bc(N, 0);
-   int64_t regBase = 0;
    for (int32_t m = 0; m < nMembers; ++m) {
       const lgpu_mesh_desc &d = members[m];
       const int32_t n0 = e->nodeStart[m], e0 = e->elemStart[m];
@@ -645,35 +647,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
       const int32_t ns[3] = {d.numSymmX, d.numSymmY, d.numSymmZ};
       for (int a = 0; a < 3; ++a)
          for (int32_t i = 0; i < ns[a]; ++i) bc[(size_t)(n0 + sy[a][i])] |= (uint8_t)(1u << a);
-      int64_t pos = (int64_t)blockStart[m] * (kEosBlock / s.eosShare);
-      // As for a single domain: the member's elements grouped by EOS repeat
-      // count, largest first, in mesh order within a group; the member's
-      // remaining region slots stay empty at its end.
-      std::vector<int32_t> repOf((size_t)d.numElem, 1), reps;
-      for (int32_t r = 0; r < d.numReg; ++r) {
-         const int32_t rep = region_rep(r, d.numReg, d.cost);
-         if (d.regElemSize[r] > 0 && std::find(reps.begin(), reps.end(), rep) == reps.end())
-            reps.push_back(rep);
-         for (int32_t i = 0; i < d.regElemSize[r]; ++i) repOf[(size_t)d.regElemlist[r][i]] = rep;
-      }
-      std::sort(reps.begin(), reps.end(), std::greater<int32_t>());
-      for (int32_t k = 0; k < d.numReg; ++k) {
-         regStart[(size_t)(regBase + k)] = (int32_t)pos;
-         regRep[(size_t)(regBase + k)] = k < (int32_t)reps.size() ? reps[(size_t)k] : 1;
-         if (k < (int32_t)reps.size())
-            for (int32_t el = 0; el < d.numElem; ++el)
-               if (repOf[(size_t)el] == reps[(size_t)k]) perm[(size_t)pos++] = el + e0;
-      }
-      regBase += d.numReg;
-      for (int32_t b = blockStart[m]; b < blockStart[m + 1]; ++b) blockMember[(size_t)b] = m;
    }
-   regStart[(size_t)numRegTot] = (int32_t)nPerm;
-   // k_eos dispatch slots: blocks in order, each with its repeat counts
-   std::vector<int32_t> blockOrder((size_t)blockStart[nMembers]);
-   for (size_t b = 0; b < blockOrder.size(); ++b) blockOrder[b] = (int32_t)b;
-   const std::vector<EosSlot> eosSlots = eos_slots(blockOrder, regStart, regRep, (int64_t)nPerm,
-                                                  s.eosShare);
-
    auto h2d = [&](void *dst, const void *src, size_t bytes) {
       return hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice) == hipSuccess;
    };
@@ -685,9 +659,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
              h2d((void *)s.elemBC, nbrs[6].data(), 4 * E) &&
              h2d((void *)s.nodeElemStart, nodeElemStart.data(), 4 * (N + 1)) &&
              (nCorner == 0 || h2d((void *)s.cornerList, corner.data(), 4 * nCorner)) &&
-             h2d((void *)s.perm, perm.data(), 4 * nPerm) &&
-             h2d((void *)s.regStart, regStart.data(), 4 * regStart.size()) &&
-             h2d((void *)s.regRep, regRep.data(), 4 * regRep.size()) &&
+             h2d((void *)s.perm, perm.data(), 4 * E) &&
              h2d((void *)s.nodeBC, bc.data(), N) &&
              h2d((void *)s.memberNodeStart, e->nodeStart.data(), 4 * e->nodeStart.size()) &&
              h2d((void *)s.memberElemStart, e->elemStart.data(), 4 * e->elemStart.size()) &&

@@ -44,10 +44,11 @@ enum ErrSite {
    kNumErrSites = 8
 };
 
-// One k_eos workgroup's perm block and its repeat counts (a block spans at
-// most two work-list groups unless a group holds fewer than a block).
+// One k_eos workgroup: `count` elements from position `pos` of the work list,
+// all with `rep` repeats, each of them shared by `share` threads (1, or
+// kEosShare in launches with k_eos's kSplit).
 struct EosSlot {
-   int32_t block, rep0, split, rep1;
+   int32_t pos, count, rep, share;
 };
 
 struct Consts {
@@ -193,7 +194,7 @@ struct MemberBrick {
 
 // Everything a cycle touches on the device.
 struct DevState {
-   int32_t numElem, numNode, numReg;
+   int32_t numElem, numNode;
    int32_t xcdRemap; // 1: map consecutive blocks onto one XCD's L2
    // node fields (current buffer; the brick path writes the other one)
    double *x, *y, *z, *xd, *yd, *zd, *nodalMass;
@@ -216,10 +217,10 @@ struct DevState {
    // corner planes: [(component*2 + kind)*8 + corner][elem], kind 0 stress, 1 hourglass
    void *corner;
    // region order
-   int32_t numPerm;         // entries of perm (>= numElem; -1 marks padding)
-   const int32_t *perm;     // region-major element order
-   const int32_t *regStart; // numReg+1 offsets into perm
-   const int32_t *regRep;   // EOS repeat count per region
+   const int32_t *perm;     // elements grouped by EOS repeat count
+   const struct EosSlot *eosSlot; // what each k_eos workgroup works on
+   int32_t eosBlocks;       // k_eos workgroups
+   int32_t eosSplit;        // some slots share elements between threads
    // control
    int32_t *err;            // kNumErrSites flags
    double *dtPartial;       // one problem: kDtSlots pairs of min_key values; ensemble: 2 per
@@ -234,13 +235,7 @@ struct DevState {
    int32_t isBrick;
    int32_t nodalBlock; // nodal pass by k_nodal_block instead of k_nodal_brick
    int32_t kinFlat;    // kinematics by k_kin_flat instead of k_kin_brick
-   int32_t brickFaces; // k_eos computes face neighbours and BC masks from the brick
-   // k_eos dispatch table (one problem): workgroup i processes perm block
-   // eosSlot[i].block, whose positions below eosSlot[i].split take repeat
-   // count rep0 and the others rep1 (rep0 < 0: look each position up in
-   // regStart).  Null (ensembles): block i, counts looked up.
-   const struct EosSlot *eosSlot;
-   int32_t eosShare; // k_eos: threads that share an element's repeats
+   int32_t brickFaces; // k_eos computes face neighbours and BC masks from the brick (or each member's)
    // Ensemble of independent problems (nMembers > 0): members are
    // concatenated; each has its own dt, loop flag and error flags.
    int32_t nMembers;
@@ -249,7 +244,7 @@ struct DevState {
    const double *memberDt;         // per-member deltatime
    const int32_t *memberActive;    // per-member loop flag
    int32_t *memberErr;             // nMembers x kNumErrSites
-   const int32_t *blockMember;     // k_eos block -> member (-1: padding)
+   const int32_t *blockMember;     // k_eos block -> member
    const int32_t *memberBlockStart; // nMembers+1: k_eos blocks of each member
    double *memberDtOut;            // 2 per member: dtcourant, dthydro
    // ensemble on the brick path (memberBrick non-null)

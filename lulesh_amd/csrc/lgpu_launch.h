@@ -18,66 +18,41 @@ constexpr int kEosBlock = 256;
 // power of two
 constexpr int kDtSlots = 256;
 
-// Threads that share an element's repeats in small k_eos launches.
+// A run of the EOS work list: the elements of one repeat count (of one
+// problem), largest count first.
+struct EosGroup {
+   int64_t pos, count;
+   int32_t rep;
+};
+
+// Threads that share an element's repeats, and the repeat count from which
+// they do, in launches that split (eos_split).
 constexpr int kEosShare = 4;
+constexpr int kEosSplitReps = 8;
 
-// Threads per element of k_eos over numElem elements in all: kEosShare up to
-// two waves per SIMD at one thread each (131,072 elements on 256 CUs).
-// Measured, one thread / kEosShare: s=8 13.0 / 7.6 us, s=30 13.9 / 10.6, s=45
-// 15.4 / 13.7, 24 mixed members of 5..24 17.2 / 12.3; above the line s=63
-// mixed (50 repeats) 26.0 / 28.5, s=64 21.3 / 27.3, s=101 49.5 / 67.  Two
-// threads: s=30 10.9, s=64 24.6; eight: s=30 10.4, s=45 17.9.
-inline int eos_share(int64_t numElem, int cus)
+// Whether k_eos shares the repeats of the heaviest elements between threads:
+// up to 2^20 elements, where a wave's 20 to 50 repeats in a row are a good part
+// of the launch.  One thread / shared: s=8 13.7 / 7.4 us, s=30 14.8 / 8.1, s=45
+// 15.6 / 11.6, s=63 mixed (50 repeats) 25.6 / 20.3, s=64 22.1 / 21.2, s=96 FMA
+// 44.7 / 43.0, s=101 50.6 / 49.9; above: 64 members, 6.0 M elements, 268 / 291,
+// s=192 299 / 341 (each sharing thread loads the operands again).
+inline bool eos_split(int64_t numElem) { return numElem <= (1 << 20); }
+
+// The workgroups of one group.
+inline void add_eos_slots(std::vector<EosSlot> &slots, const EosGroup &g, bool split)
 {
-   return numElem <= (int64_t)cus * 4 * 64 * 2 ? kEosShare : 1;
+   const int share = split && g.rep >= kEosSplitReps ? kEosShare : 1, per = kEosBlock / share;
+   for (int64_t at = 0; at < g.count; at += per)
+      slots.push_back(EosSlot{(int32_t)(g.pos + at), (int32_t)std::min<int64_t>(per, g.count - at),
+                              g.rep, share});
 }
 
-// Workgroups of k_eos over numElem list positions.
-inline unsigned eos_blocks(int numElem, int share)
+// EOS repeat count of region r (0-based), lulesh.cc:2390-2400.
+inline int32_t region_rep(int32_t r, int32_t numReg, int32_t cost)
 {
-   const int per = kEosBlock / share;
-   return (unsigned)((numElem + per - 1) / per);
-}
-
-// k_eos dispatch slots for the perm blocks in `order`: each block's repeat
-// counts from the work-list groups (regStart: nGroups+1 perm positions,
-// possibly empty groups; regRep: nGroups counts) -- its first position's
-// group and, where the block reaches into it, the next non-empty group.  A
-// block over three or more groups gets rep0 = -1 (k_eos searches regStart).
-inline std::vector<EosSlot> eos_slots(const std::vector<int32_t> &order,
-                                      const std::vector<int32_t> &regStart,
-                                      const std::vector<int32_t> &regRep, int64_t numPositions,
-                                      int share)
-{
-   const int ng = (int)regRep.size(), per = kEosBlock / share;
-   auto group_of = [&](int64_t p) {
-      const int g = (int)(std::upper_bound(regStart.begin(), regStart.begin() + ng, (int32_t)p) -
-                          regStart.begin()) - 1;
-      // the last group starting at or before p: of several groups that start
-      // at p, the last, which is the one holding p where any does (empty
-      // groups only precede it, or cover padding after a member's elements)
-      return std::max(0, g);
-   };
-   std::vector<EosSlot> slots(order.size());
-   for (size_t i = 0; i < order.size(); ++i) {
-      const int64_t p0 = (int64_t)order[i] * per;
-      const int64_t p1 = std::max(p0, std::min<int64_t>(p0 + per, numPositions) - 1);
-      EosSlot &sl = slots[i];
-      sl.block = order[i];
-      const int g0 = group_of(p0), g1 = group_of(p1);
-      if (g0 == g1) {
-         sl.rep0 = sl.rep1 = regRep[(size_t)g0];
-         sl.split = (int32_t)(p0 + per);
-      } else if (group_of(regStart[(size_t)g0 + 1]) == g1) {
-         sl.rep0 = regRep[(size_t)g0];
-         sl.rep1 = regRep[(size_t)g1];
-         sl.split = regStart[(size_t)g0 + 1];
-      } else {
-         sl.rep0 = -1;
-         sl.split = sl.rep1 = 0;
-      }
-   }
-   return slots;
+   if (r < numReg / 2) return 1;
+   if (r < numReg - (numReg + 15) / 20) return 1 + cost;
+   return 10 * (1 + cost);
 }
 
 template <class P>
