@@ -20,6 +20,7 @@
 #include "lgpu_brick.h"
 #include "lgpu_kernels.h"
 #include "lgpu_launch.h"
+#include "lgpu_time.h"
 #include "lulesh_gpu.h"
 
 using namespace lgpu;
@@ -36,54 +37,14 @@ const char *const kEnsKernelNames[kENumKernels] = {"k_force", "k_node", "k_kin",
 constexpr size_t kAlign = 256;
 inline size_t align_up(size_t v) { return (v + kAlign - 1) & ~(kAlign - 1); }
 
-// Per-member time state, struct of arrays (the kernels read deltatime and
-// active as plain arrays).
-struct EnsTime {
-   double *time, *deltatime, *dtcourant, *dthydro, *stoptime, *dtfixed, *dtmax, *multlb, *multub;
-   int32_t *cycle, *active;
-   // the run's cycle limit, one value in device memory: set by each
-   // lgpu_ensemble_run, so that the cycle graphs do not depend on it
-   int32_t *maxCycle;
-};
-
-// TimeIncrement per member (lulesh.cc:166-222) and the loop test of
-// lulesh.cc:2745; a member whose step failed stops.
+// TimeIncrement per member (lulesh.cc:166-222) of a run's first cycle; later
+// ones run at the end of the cycle before (k_dt_reduce).
 __global__ void k_time_increment_ens(EnsTime t, const double *dtOut, const int32_t *err,
                                      int nMembers)
 {
    const int m = blockIdx.x * blockDim.x + threadIdx.x;
-   if (m >= nMembers || !t.active[m]) return;
-   const int maxCycle = *t.maxCycle;
-   bool failed = false;
-   for (int i = 0; i < kNumErrSites; ++i) failed = failed || (err[m * kNumErrSites + i] != 0);
-   if (t.cycle[m] > 0) {
-      t.dtcourant[m] = dtOut[2 * m];
-      t.dthydro[m] = dtOut[2 * m + 1];
-   }
-   if (failed || !(t.time[m] < t.stoptime[m] && t.cycle[m] < maxCycle)) {
-      t.active[m] = 0;
-      return;
-   }
-   double targetdt = t.stoptime[m] - t.time[m];
-   double dt = t.deltatime[m];
-   if (t.dtfixed[m] <= 0.0 && t.cycle[m] != 0) {
-      const double olddt = dt;
-      double newdt = 1.0e+20;
-      if (t.dtcourant[m] < newdt) newdt = t.dtcourant[m] / 2.0;
-      if (t.dthydro[m] < newdt) newdt = t.dthydro[m] * 2.0 / 3.0;
-      const double ratio = newdt / olddt;
-      if (ratio >= 1.0) {
-         if (ratio < t.multlb[m]) newdt = olddt;
-         else if (ratio > t.multub[m]) newdt = olddt * t.multub[m];
-      }
-      if (newdt > t.dtmax[m]) newdt = t.dtmax[m];
-      dt = newdt;
-   }
-   if (targetdt > dt && targetdt < 4.0 * dt / 3.0) targetdt = 2.0 * dt / 3.0;
-   if (targetdt < dt) dt = targetdt;
-   t.deltatime[m] = dt;
-   t.time[m] += dt;
-   t.cycle[m] += 1;
+   if (m >= nMembers) return;
+   time_increment(t, m, dtOut[2 * m], dtOut[2 * m + 1], any_error(err + m * kNumErrSites));
 }
 
 } // namespace
@@ -154,8 +115,6 @@ void swap_nodes(lgpu_ensemble *e)
 template <class P>
 void launch_cycle(lgpu_ensemble *e)
 {
-   hipLaunchKernelGGL(k_time_increment_ens, dim3((e->nMembers + 63) / 64), dim3(64), 0, e->stream,
-                      e->t, e->s.memberDtOut, e->s.memberErr, e->nMembers);
    if (e->brick) {
       Launch<P>::nodal_brick_members(e->s, e->k, e->nodalBlocks, e->stream);
       swap_nodes(e);
@@ -186,8 +145,6 @@ int timed_cycle(lgpu_ensemble *e, float ms[kENumKernels])
    hipEvent_t ev[kENumKernels + 1];
    for (auto &x : ev) ENS_HIP(e, hipEventCreate(&x));
    ENS_HIP(e, hipEventRecord(ev[0], e->stream));
-   hipLaunchKernelGGL(k_time_increment_ens, dim3((e->nMembers + 63) / 64), dim3(64), 0, e->stream,
-                      e->t, e->s.memberDtOut, e->s.memberErr, e->nMembers);
    ENS_HIP(e, hipEventRecord(ev[1], e->stream));
    if (e->brick) {
       Launch<P>::nodal_brick_members(e->s, e->k, e->nodalBlocks, e->stream);
@@ -626,6 +583,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    s.nMembers = nMembers;
    s.memberDt = t.deltatime;
    s.memberActive = t.active;
+   s.ensTime = t;
 
    // Concatenated connectivity.
    std::vector<int32_t> nodelist(8 * E), nbrs[7], nodeElemStart(N + 1), corner(nCorner);
@@ -775,8 +733,18 @@ int lgpu_ensemble_run(lgpu_ensemble *e, lgpu_time_state *ts, int32_t maxCycle, i
       const int r = build_graph(e);
       if (r) return r;
    }
-   const int batch = 8;
-   for (;;) {
+   hipLaunchKernelGGL(k_time_increment_ens, dim3((unsigned)((M + 63) / 64)), dim3(64), 0, e->stream,
+                      e->t, e->s.memberDtOut, e->s.memberErr, M);
+   ENS_HIP(e, hipGetLastError());
+   // Cycles are enqueued in batches between host checks of the loop flags, and
+   // no more of them than the member with the most cycles left can run: only
+   // a run that ends at stoptime (or on an error) enqueues no-op cycles.
+   int64_t remaining = 0;
+   for (int m = 0; m < M; ++m)
+      remaining = std::max<int64_t>(remaining, (int64_t)maxCycle - ts[m].cycle);
+   while (remaining > 0) {
+      const int batch = (int)std::min<int64_t>(8, remaining);
+      remaining -= batch;
       for (int b = 0; b < batch; ++b) {
          if (e->timing) {
             float ms[kENumKernels];

@@ -192,6 +192,22 @@ struct MemberBrick {
    int32_t nodeOff, elemOff, nodalBlock0, kinBlock0;
 };
 
+// Per-member time state of an ensemble, struct of arrays (the kernels read
+// deltatime and active as plain arrays).
+struct EnsTime {
+   double *time, *deltatime, *dtcourant, *dthydro, *stoptime, *dtfixed, *dtmax, *multlb, *multub;
+   int32_t *cycle, *active;
+   // the run's cycle limit, one value in device memory: set by each
+   // lgpu_ensemble_run, so that the cycle graphs do not depend on it
+   int32_t *maxCycle;
+};
+
+// Results of a cycle in pinned host memory, for lgpu_time_constraints.
+struct HostOut {
+   double dt[2];
+   int32_t err[kNumErrSites];
+};
+
 // Everything a cycle touches on the device.
 struct DevState {
    int32_t numElem, numNode;
@@ -226,6 +242,7 @@ struct DevState {
    double *dtPartial;       // one problem: kDtSlots pairs of min_key values; ensemble: 2 per
                             // k_eos block
    double *dtOut;           // [0] dtcourant, [1] dthydro
+   HostOut *hostOut;        // one problem, host-driven: the results again (or null)
    const double *dtDevice;  // device-side deltatime (null: use argument)
    const int32_t *active;   // device-side loop flag (null: always active)
    // device-side time state: k_dt_slots also runs the next cycle's
@@ -247,6 +264,7 @@ struct DevState {
    const int32_t *blockMember;     // k_eos block -> member
    const int32_t *memberBlockStart; // nMembers+1: k_eos blocks of each member
    double *memberDtOut;            // 2 per member: dtcourant, dthydro
+   EnsTime ensTime;                // the members' next TimeIncrement
    // ensemble on the brick path (memberBrick non-null)
    const MemberBrick *memberBrick;
    const int32_t *nodalBlockMember; // k_nodal_brick workgroup -> member

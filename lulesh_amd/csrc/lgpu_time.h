@@ -1,5 +1,5 @@
 // lgpu_time.h -- device-side time state and TimeIncrement (lulesh.cc:166-222)
-// of the device loop (lgpu_run).
+// of the device loops (lgpu_run, lgpu_ensemble_run).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -16,13 +16,11 @@ struct DevTime {
 
 // TimeIncrement (lulesh.cc:166-222) at the top of a cycle, given the dt
 // constraints of the cycle before (used when cycle > 0); also decides whether
-// the cycle runs at all (the loop test of lulesh.cc:2745, and an error flag
-// of the cycle before ends the loop).  One thread.
-__device__ inline void time_increment(DevTime *t, double dtc, double dth, const int32_t *err)
+// the cycle runs at all (the loop test of lulesh.cc:2745; failed: an error
+// flag of the cycle before ends the loop).  One thread.
+__device__ inline void time_increment(DevTime *t, double dtc, double dth, bool failed)
 {
    if (!t->active) return;
-   bool failed = false;
-   for (int i = 0; i < kNumErrSites; ++i) failed = failed || (err[i] != 0);
    if (t->cycle > 0) {
       t->dtcourant = dtc;
       t->dthydro = dth;
@@ -50,6 +48,28 @@ __device__ inline void time_increment(DevTime *t, double dtc, double dth, const 
    if (targetdt < t->deltatime) t->deltatime = targetdt;
    t->time += t->deltatime;
    t->cycle += 1;
+}
+
+__device__ inline bool any_error(const int32_t *err)
+{
+   bool failed = false;
+   for (int i = 0; i < kNumErrSites; ++i) failed = failed || (err[i] != 0);
+   return failed;
+}
+
+// The same for member m of an ensemble.
+__device__ inline void time_increment(const EnsTime &t, int m, double dtc, double dth, bool failed)
+{
+   DevTime d{t.time[m],    t.deltatime[m], t.dtcourant[m], t.dthydro[m], t.stoptime[m],
+             t.dtfixed[m], t.dtmax[m],     t.multlb[m],    t.multub[m],  t.cycle[m],
+             *t.maxCycle,  t.active[m],    0};
+   time_increment(&d, dtc, dth, failed);
+   t.time[m] = d.time;
+   t.deltatime[m] = d.deltatime;
+   t.dtcourant[m] = d.dtcourant;
+   t.dthydro[m] = d.dthydro;
+   t.cycle[m] = d.cycle;
+   t.active[m] = d.active;
 }
 
 } // namespace lgpu
