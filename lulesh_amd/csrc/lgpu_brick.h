@@ -126,6 +126,31 @@ inline int pick_brick_chunk(const Brick &g, int slots, int least)
    return pick_chunk((int64_t)g.tilesX * g.tilesY, g.en, slots, least, 8);
 }
 
+// The chunk for launches of several rounds whose workgroups end at different
+// times (the mixed form, 3 a CU; ensembles, whose members' last chunks are
+// shorter): least work per resident workgroup, plus half a walk for the tail
+// of the launch.  columns[i] column tiles of planes[i] planes each.  Mixed:
+// s=192 chunk 22 -> 13, 412 -> 401 us; s=160 22 -> 7, 276 -> 242; s=128 15 ->
+// 5, 138 -> 133 (fewest rounds against this).
+inline int pick_tail_chunk(const std::vector<int64_t> &columns, const std::vector<int> &planes,
+                           int slots, int fallback)
+{
+   if (slots < 1) return fallback;
+   int best = fallback;
+   double bestWork = 1e300;
+   for (int ch = 1; ch <= 64; ++ch) {
+      double walked = 0.;
+      for (size_t i = 0; i < columns.size(); ++i)
+         walked += (double)columns[i] * (planes[i] + (planes[i] + ch - 1) / ch);
+      const double work = std::max(walked / slots + 0.5 * (ch + 1), ch + 1.0);
+      if (work < bestWork) {
+         bestWork = work;
+         best = ch;
+      }
+   }
+   return best;
+}
+
 inline void set_kin_chunk(Brick &g, int chunk)
 {
    g.kinChunk = std::max(1, std::min(chunk, g.s));

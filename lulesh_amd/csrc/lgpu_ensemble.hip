@@ -240,9 +240,7 @@ int launch_graph(lgpu_ensemble *e)
 }
 
 // The brick path's default kernels and nodal chunk.  A walk's cost is taken
-// over all members' workgroups; within it the chunk with the least work per
-// resident workgroup, plus half a walk for the tail of the launch (the
-// members' last chunks are shorter, so rounds do not end together).  64
+// over all members' workgroups.  64
 // members of 16..64, FP64: chunk 10, 500 us (7: 495, 4: 519); 30 of 10..40:
 // chunk 4, 68.7 us (8: 81.8, k_nodal_block 84.8); 24 of 5..24: k_nodal_block,
 // FP64 18.6 and mixed 13.6 us (best walk 24.1 and 18.5).
@@ -270,21 +268,18 @@ void pick_brick_kernels(lgpu_ensemble *e)
    }
    e->s.kinFlat = largest <= kKinFlatMax;
    if (slots < 1) return;
+   std::vector<int64_t> columns;
+   std::vector<int> planes;
+   for (const Brick &g : bricks) {
+      columns.push_back((int64_t)g.tilesX * g.tilesY);
+      planes.push_back(g.en);
+   }
+   e->nodalChunk = pick_tail_chunk(columns, planes, slots, e->nodalChunk);
    int64_t least = INT64_MAX;
-   double best = 1e300;
    for (int ch = 1; ch <= 22; ++ch) {
-      int64_t walks = 0, planes = 0;
-      for (const Brick &g : bricks) {
-         const int64_t chunks = (g.en + ch - 1) / ch;
-         walks += (int64_t)g.tilesX * g.tilesY * chunks;
-         planes += (int64_t)g.tilesX * g.tilesY * (g.en + chunks);
-      }
+      int64_t walks = 0;
+      for (const Brick &g : bricks) walks += (int64_t)g.tilesX * g.tilesY * ((g.en + ch - 1) / ch);
       least = std::min(least, (walks + slots - 1) / slots * (ch + 1));
-      const double work = std::max((double)planes / slots + 0.5 * (ch + 1), ch + 1.0);
-      if (work < best) {
-         best = work;
-         e->nodalChunk = ch;
-      }
    }
    e->s.nodalBlock = block_is_faster(blocks, slots, least);
 }

@@ -98,10 +98,13 @@ struct PolicyFp64 {
    // 416 -> 411 us; FP64 582 -> 600 us, FMA 505 -> 534 us (the stress work
    // then waits for every load at once)
    static constexpr bool kPinElemFields = false;
-   // brick kernel: load the next element plane's coordinates and fields in
-   // the node phase of the current one (between its barriers).  FP64_FMA
-   // s=192: 498 -> 486 us; FP64 no gain (255 VGPRs)
-   static constexpr bool kPrefetchElem = false;
+   // brick kernel: carry an element's upper corners to the next plane in
+   // registers, and load the next plane's other corners and fields in the
+   // node phase of the current one.  s=192: FP64 555 -> 507 us, FP64_FMA 473 ->
+   // 438 (all eight corners loaded there instead, the FMA form's way before:
+   // FP64 534), s=101 FP64 90.4 -> 85.8; mixed spills 12 registers at 3
+   // waves/SIMD (s=192 410 -> 527 us)
+   static constexpr bool kCarryPlane = true;
    // k_eos waves per SIMD: FP64 at 7 (at most 72 VGPRs); 8 (64 VGPRs, four
    // spilled) ran 326 -> 332 us at s=192
    static constexpr int kEosWaves = 7;
@@ -118,7 +121,6 @@ struct PolicyFp64 {
 // translation unit); the types are those of PolicyFp64.
 struct PolicyFp64Fma : PolicyFp64 {
    static constexpr bool kHgVelEarly = true;
-   static constexpr bool kPrefetchElem = true;
 };
 
 struct PolicyMixed {
@@ -137,7 +139,7 @@ struct PolicyMixed {
    static constexpr bool kOffset32 = true;
    static constexpr bool kHgVelEarly = true;
    static constexpr bool kPinElemFields = true;
-   static constexpr bool kPrefetchElem = false; // 56 spills at 3 waves/SIMD
+   static constexpr bool kCarryPlane = false;
    // k_eos at 8 waves per SIMD (at most 64 VGPRs): 214 -> 211 us at s=192
    static constexpr int kEosWaves = 8;
    static constexpr bool kNodePhasePrio = false;
