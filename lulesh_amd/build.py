@@ -44,6 +44,7 @@ HIP_SOURCES = {
     "lgpu_ensemble.hip": ["-ffp-contract=off"],
     "lgpu_setup.hip": ["-ffp-contract=off"],
     "lgpu_noalloc.hip": ["-ffp-contract=off"],
+    "lgpu_convert.hip": ["-ffp-contract=off"],
 }
 HOST_SOURCES = ["host/domain.cc", "host/glibc_rand.cc", "host/viz.cc"]
 

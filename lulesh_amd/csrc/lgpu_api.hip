@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "lgpu_brick.h"
+#include "lgpu_convert.h"
 #include "lgpu_kernels.h"
 #include "lgpu_launch.h"
 #include "lgpu_setup.h"
@@ -291,6 +292,13 @@ double *real_field_ptr(lgpu_ctx *c, int f, bool &isElem, bool &narrow)
    case LGPU_DELV_ZETA: return static_cast<double *>(s.delv_zeta);
    default: return nullptr;
    }
+}
+
+// Device scratch of numElem doubles that nothing holds between cycles: the
+// node buffer the next cycle writes (brick), or the corner planes.
+double *scratch_doubles(lgpu_ctx *c)
+{
+   return c->s.isBrick ? c->s.xo : static_cast<double *>(c->s.corner);
 }
 
 int enable_diagnostics(lgpu_ctx *c)
@@ -862,7 +870,12 @@ int lgpu_upload(lgpu_ctx *c, int field, const double *host)
    if (!dst) return LGPU_EINVAL;
    const size_t n = isElem ? (size_t)c->numElem : (size_t)c->numNode;
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
-   if (narrow) {
+   if (narrow && (int64_t)n > kConvertOnHost) {
+      double *wide = scratch_doubles(c);
+      HIP_OR_RETURN(c, hipMemcpy(wide, host, sizeof(double) * n, hipMemcpyHostToDevice));
+      HIP_OR_RETURN(c, launch_narrow(wide, reinterpret_cast<float *>(dst), (int64_t)n, c->stream));
+      HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
+   } else if (narrow) {
       std::vector<float> tmp(n);
       for (size_t i = 0; i < n; ++i) tmp[i] = (float)host[i];
       HIP_OR_RETURN(c, hipMemcpy(dst, tmp.data(), sizeof(float) * n, hipMemcpyHostToDevice));
@@ -883,7 +896,12 @@ int lgpu_download(lgpu_ctx *c, int field, double *host)
       std::fill(host, host + n, 0.0);
       return LGPU_OK;
    }
-   if (narrow) {
+   if (narrow && (int64_t)n > kConvertOnHost) {
+      double *wide = scratch_doubles(c);
+      HIP_OR_RETURN(c, launch_widen(reinterpret_cast<const float *>(src), wide, (int64_t)n, c->stream));
+      HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
+      HIP_OR_RETURN(c, hipMemcpy(host, wide, sizeof(double) * n, hipMemcpyDeviceToHost));
+   } else if (narrow) {
       std::vector<float> tmp(n);
       HIP_OR_RETURN(c, hipMemcpy(tmp.data(), src, sizeof(float) * n, hipMemcpyDeviceToHost));
       for (size_t i = 0; i < n; ++i) host[i] = (double)tmp[i];

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "lgpu_brick.h"
+#include "lgpu_convert.h"
 #include "lgpu_kernels.h"
 #include "lgpu_launch.h"
 #include "lgpu_time.h"
@@ -371,6 +372,13 @@ double *field_base(lgpu_ensemble *e, int f, bool &isElem, bool &narrow)
    }
 }
 
+// Device scratch of a member's elements in doubles that nothing holds between
+// cycles, as for a single problem.
+double *scratch_doubles(lgpu_ensemble *e)
+{
+   return e->brick ? e->s.xo : static_cast<double *>(e->s.corner);
+}
+
 } // namespace
 
 extern "C" {
@@ -652,7 +660,12 @@ int lgpu_ensemble_upload(lgpu_ensemble *e, int32_t member, int field, const doub
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
    ENS_HIP(e, hipStreamSynchronize(e->stream));
-   if (narrow) {
+   if (narrow && (int64_t)n > kConvertOnHost) {
+      double *wide = scratch_doubles(e);
+      ENS_HIP(e, hipMemcpy(wide, host, 8 * n, hipMemcpyHostToDevice));
+      ENS_HIP(e, launch_narrow(wide, reinterpret_cast<float *>(base) + off, (int64_t)n, e->stream));
+      ENS_HIP(e, hipStreamSynchronize(e->stream));
+   } else if (narrow) {
       std::vector<float> tmp(n);
       for (size_t i = 0; i < n; ++i) tmp[i] = (float)host[i];
       ENS_HIP(e, hipMemcpy(reinterpret_cast<float *>(base) + off, tmp.data(), 4 * n, hipMemcpyHostToDevice));
@@ -671,7 +684,12 @@ int lgpu_ensemble_download(lgpu_ensemble *e, int32_t member, int field, double *
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
    ENS_HIP(e, hipStreamSynchronize(e->stream));
-   if (narrow) {
+   if (narrow && (int64_t)n > kConvertOnHost) {
+      double *wide = scratch_doubles(e);
+      ENS_HIP(e, launch_widen(reinterpret_cast<const float *>(base) + off, wide, (int64_t)n, e->stream));
+      ENS_HIP(e, hipStreamSynchronize(e->stream));
+      ENS_HIP(e, hipMemcpy(host, wide, 8 * n, hipMemcpyDeviceToHost));
+   } else if (narrow) {
       std::vector<float> tmp(n);
       ENS_HIP(e, hipMemcpy(tmp.data(), reinterpret_cast<float *>(base) + off, 4 * n, hipMemcpyDeviceToHost));
       for (size_t i = 0; i < n; ++i) host[i] = tmp[i];
