@@ -62,6 +62,7 @@ struct lgpu_ctx {
    std::vector<PlacedSlot> eosSlots; // in work-list order
    int eosInterleave = 0;
    int32_t brickPerCu = 0;
+   int64_t brickSlots = 0, genericSlots = 0; // resident workgroups: nodal brick kernels, k_force
    bool timing = false;
    uint32_t timingMask = 0xffffffffu;
    Consts k{};
@@ -349,7 +350,8 @@ int launch_elements(lgpu_ctx *c, double dt)
    if (r) return r;
    r = timed(c, kKEos, [&] { Launch<P>::eos(c->s, c->k, c->stream); });
    if (r) return r;
-   c->hostOutFresh = !c->s.time;
+   c->hostOutFresh = !c->s.timeIn;
+   if (c->s.timeIn) return LGPU_OK; // the dt slots are folded as the next cycle begins
    return timed(c, kKDtReduce, [&] { Launch<P>::dt_reduce(c->s, c->stream); });
 }
 
@@ -359,24 +361,6 @@ int resolve_status(const int32_t *err)
    if (err[kErrQStop]) return LGPU_QSTOP_ERROR;
    if (err[kErrMaterialV]) return LGPU_VOLUME_ERROR;
    return LGPU_OK;
-}
-
-// TimeIncrement for the first cycle of a device-side loop; later cycles'
-// increments are folded into the dt reduction, k_dt_slots (lgpu_time.h).
-__global__ void k_time_increment(DevTime *t, const double *dtOut, const int32_t *err)
-{
-   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-   time_increment(t, dtOut[0], dtOut[1], any_error(err));
-}
-
-// Folds the last cycle's dt results into the time state once the loop ends.
-__global__ void k_time_final(DevTime *t, const double *dtOut)
-{
-   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-   if (t->cycle > 0) {
-      t->dtcourant = dtOut[0];
-      t->dthydro = dtOut[1];
-   }
 }
 
 // What the context's arena and kernel path depend on.
@@ -456,10 +440,12 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    if (!brick) add(&s.corner, cornerBytes * (size_t)plane * 48);
    add((void **)&s.perm, sizeof(int32_t) * E);
    add((void **)&s.eosSlot, sizeof(EosSlot) * eosBlocks);
-   add((void **)&s.err, sizeof(int32_t) * kNumErrSites);
-   add((void **)&s.dtPartial, sizeof(double) * 2 * kDtSlots);
+   // two sets each, which the cycles of a device loop use in turn (set 0 by
+   // host-driven cycles)
+   add((void **)&s.err, 2 * sizeof(int32_t) * kNumErrSites);
+   add((void **)&s.dtPartial, 2 * sizeof(double) * 2 * kDtSlots);
    add((void **)&s.dtOut, sizeof(double) * 2);
-   add((void **)&c->devTime, sizeof(DevTime));
+   add((void **)&c->devTime, 2 * sizeof(DevTime));
    size_t total = 0;
    for (const Slot &sl : slots) total += sl.bytes;
    if (hipMalloc((void **)&c->arena, total) != hipSuccess) {
@@ -474,14 +460,14 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
       *sl.dst = c->arena + off;
       off += sl.bytes;
    }
-   // the dt slot pairs start at the key of 1.0e+20 (k_dt_slots resets them
-   // to it after every read): sign bit set on the value's bits
+   // the dt slot pairs start at the key of 1.0e+20 (they go back to it after
+   // every read): sign bit set on the value's bits
    {
       const double big = 1.0e+20;
       uint64_t key = 0;
       std::memcpy(&key, &big, sizeof key);
       key |= 0x8000000000000000ull;
-      const std::vector<uint64_t> init(2 * (size_t)kDtSlots, key);
+      const std::vector<uint64_t> init(4 * (size_t)kDtSlots, key);
       if (hipMemcpy(s.dtPartial, init.data(), sizeof(uint64_t) * init.size(), hipMemcpyHostToDevice) !=
           hipSuccess)
          return fail(LGPU_EDEVICE);
@@ -490,6 +476,7 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    s.numNode = sp.numNode;
    s.xcdRemap = 1;
    s.isBrick = brick ? 1 : 0;
+   c->genericSlots = (int64_t)cus * 2;
    s.brickFaces = (brick && sp.brickFaces) ? 1 : 0;
    if (brick) {
       Brick &g = s.brick;
@@ -501,6 +488,7 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
       default: perCu = Launch<PolicyFp64>::nodal_brick_blocks_per_cu(); break;
       }
       c->brickPerCu = perCu;
+      c->brickSlots = (int64_t)cus * perCu;
       const int slots = cus * perCu; // k_nodal_block has the walk's occupancy
       set_brick_chunk(g, pick_brick_chunk(g, slots, 1));
       s.nodalBlock = slots > 0 && block_is_faster(block_blocks(g), slots,
@@ -968,60 +956,81 @@ int lgpu_run(lgpu_ctx *c, lgpu_time_state *ts, int32_t maxCycle)
    h->cycle = ts->cycle;
    h->maxCycle = maxCycle;
    h->active = 1;
-   h->pad = 0;
-   HIP_OR_RETURN(c, hipMemcpyAsync(c->devTime, h, sizeof(DevTime), hipMemcpyHostToDevice, c->stream));
+   h->fresh = 1;
+   DevTime *const times = c->devTime;
+   double *const slots = c->s.dtPartial;
+   int32_t *const errs = c->s.err;
+   HIP_OR_RETURN(c, hipMemcpyAsync(times, h, sizeof(DevTime), hipMemcpyHostToDevice, c->stream));
    c->hostOutFresh = false;
-   // dtOut feeds the first TimeIncrement only when cycle > 0: seed it with
-   // the caller's constraints.
+   // dtOut holds the caller's constraints until a cycle has run.
    c->hostDt[0] = ts->dtcourant;
    c->hostDt[1] = ts->dthydro;
    HIP_OR_RETURN(c, hipMemcpyAsync(c->s.dtOut, c->hostDt, sizeof(double) * 2,
                                    hipMemcpyHostToDevice, c->stream));
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
 
-   c->s.dtDevice = &c->devTime->deltatime;
-   c->s.active = &c->devTime->active;
-   c->s.time = c->devTime; // k_dt_slots runs the next cycle's TimeIncrement
+   const bool fold = c->s.isBrick
+                        ? c->s.nodalBlock && fold_start(block_blocks(c->s.brick), c->brickSlots)
+                        : fold_start((c->numElem + c->block - 1) / c->block, c->genericSlots);
+   // Cycle j reads the time state, error flags and dt slots of set j mod 2 and
+   // writes the other set.
+   auto use_sets = [&](int j) {
+      const int in = j & 1, out = in ^ 1;
+      DevState &s = c->s;
+      s.timeIn = times + in;
+      s.timeOut = times + out;
+      s.errPrev = errs + in * kNumErrSites;
+      s.err = errs + out * kNumErrSites;
+      s.dtPartialPrev = slots + in * 2 * kDtSlots;
+      s.dtPartial = slots + out * 2 * kDtSlots;
+      s.startFold = fold ? 1 : 0;
+      s.dtDevice = &s.timeOut->deltatime;
+      s.active = &s.timeOut->active;
+   };
    // Cycles are enqueued in batches between host checks of the loop flag.
    // No more cycles are enqueued than the cycle limit allows, so only a run
    // that ends at stoptime (or on an error) enqueues no-op cycles.
-   int64_t remaining = (int64_t)maxCycle - (int64_t)ts->cycle;
-   int st = LGPU_OK;
-   bool first = true;
-   for (;;) {
-      const int batch = (int)std::max<int64_t>(1, std::min<int64_t>(16, remaining));
+   int64_t remaining = std::max<int64_t>(1, (int64_t)maxCycle - (int64_t)ts->cycle);
+   int st = LGPU_OK, done = 0;
+   while (remaining > 0 && !st) {
+      const int batch = (int)std::min<int64_t>(16, remaining);
       remaining -= batch;
-      for (int b = 0; b < batch; ++b) {
-         if (first) {
-            st = timed(c, kKTimeIncrement, [&] {
-               hipLaunchKernelGGL(k_time_increment, dim3(1), dim3(64), 0, c->stream, c->devTime,
-                                  c->s.dtOut, c->s.err);
-            });
-            if (st) break;
-            first = false;
-         }
-         st = lgpu_lagrange_nodal(c, 0.0);
-         if (st) break;
-         st = lgpu_lagrange_elements(c, 0.0);
-         if (st) break;
+      for (int b = 0; b < batch && !st; ++b) {
+         use_sets(done);
+         done ^= 1;
+         if (!fold) st = timed(c, kKTimeIncrement, [&] { Launch<PolicyFp64>::begin(c->s, c->stream); });
+         if (!st) st = lgpu_lagrange_nodal(c, 0.0);
+         if (!st) st = lgpu_lagrange_elements(c, 0.0);
       }
+      if (st || remaining <= 0) break;
+      st = set_hip_error(c, hipMemcpyAsync(h, c->s.timeOut, sizeof(DevTime), hipMemcpyDeviceToHost,
+                                           c->stream), "hipMemcpyAsync");
+      if (!st) st = set_hip_error(c, hipStreamSynchronize(c->stream), "hipStreamSynchronize");
       if (st) break;
-      HIP_OR_RETURN(c, hipMemcpyAsync(h, c->devTime, sizeof(DevTime), hipMemcpyDeviceToHost, c->stream));
-      HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
       if (c->timing) harvest_timing(c);
       if (!h->active) break;
    }
+   DevTime *const last = c->s.timeOut;
+   if (!st) {
+      Launch<PolicyFp64>::run_end(c->s, slots, errs, c->stream);
+      st = set_hip_error(c, hipGetLastError(), "k_run_end");
+   }
    // Back to host-driven dt (the node buffers keep whatever swaps happened).
+   c->s.timeIn = nullptr;
+   c->s.startFold = 0;
+   c->s.timeOut = nullptr;
+   c->s.errPrev = nullptr;
+   c->s.dtPartialPrev = nullptr;
+   c->s.err = errs;
+   c->s.dtPartial = slots;
    c->s.dtDevice = nullptr;
    c->s.active = nullptr;
-   c->s.time = nullptr;
    if (st) return st;
-   hipLaunchKernelGGL(k_time_final, dim3(1), dim3(64), 0, c->stream, c->devTime, c->s.dtOut);
-   HIP_OR_RETURN(c, hipGetLastError());
-   HIP_OR_RETURN(c, hipMemcpyAsync(h, c->devTime, sizeof(DevTime), hipMemcpyDeviceToHost, c->stream));
+   HIP_OR_RETURN(c, hipMemcpyAsync(h, last, sizeof(DevTime), hipMemcpyDeviceToHost, c->stream));
    HIP_OR_RETURN(c, hipMemcpyAsync(c->hostErr, c->s.err, sizeof(int32_t) * kNumErrSites,
                                    hipMemcpyDeviceToHost, c->stream));
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
+   if (c->timing) harvest_timing(c);
    ts->time = h->time;
    ts->deltatime = h->deltatime;
    ts->dtcourant = h->dtcourant;

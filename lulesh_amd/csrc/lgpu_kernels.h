@@ -244,12 +244,17 @@ struct DevState {
    double *dtPartial;       // one problem: kDtSlots pairs of min_key values; ensemble: 2 per
                             // k_eos block
    double *dtOut;           // [0] dtcourant, [1] dthydro
+   // Device loop (null otherwise): a cycle begins with timeOut made from
+   // timeIn, the error flags and the dt slots of the cycle before (begin_cycle
+   // in lgpu_step.inc), and sets err and dtPartial itself.
+   int32_t startFold; // by the cycle's first kernel, not a launch of its own
+   const struct DevTime *timeIn;
+   struct DevTime *timeOut;
+   const int32_t *errPrev;
+   double *dtPartialPrev;
    HostOut *hostOut;        // one problem, host-driven: the results again (or null)
    const double *dtDevice;  // device-side deltatime (null: use argument)
    const int32_t *active;   // device-side loop flag (null: always active)
-   // device-side time state: k_dt_slots also runs the next cycle's
-   // TimeIncrement (null: host-driven time stepping)
-   struct DevTime *time;
    Brick brick;             // valid when isBrick
    int32_t isBrick;
    int32_t nodalBlock; // nodal pass by k_nodal_block instead of k_nodal_brick

@@ -47,6 +47,14 @@ inline void add_eos_slots(std::vector<EosSlot> &slots, const EosGroup &g, bool s
                               g.rep, share});
 }
 
+// Whether a device-loop cycle begins in its first kernel (k_nodal_block or
+// k_force, of `blocks` workgroups on `slots` resident ones) instead of
+// k_begin_cycle, a launch of 3.0 to 4.7 us.  Each workgroup then starts about
+// 1 us later, so the gain is gone after a few rounds.  Launch / first kernel,
+// us a cycle, FP64: s=8 24.6 / 21.5, s=30 25.8 / 24.1, s=45 40.1 / 39.1, s=64
+// gathers (2 rounds) 68.8 / 68.8; k_nodal_brick s=101 4.7 less and 5.5 more.
+inline bool fold_start(int64_t blocks, int64_t slots) { return blocks <= 2 * slots; }
+
 // EOS repeat count of region r (0-based), lulesh.cc:2390-2400.
 inline int32_t region_rep(int32_t r, int32_t numReg, int32_t cost)
 {
@@ -75,6 +83,10 @@ struct Launch {
    static void kin_brick_members(const DevState &s, const Consts &k, unsigned grid, hipStream_t st);
    static void eos(const DevState &s, const Consts &k, hipStream_t st);
    static void dt_reduce(const DevState &s, hipStream_t st);
+   // start of a device-loop cycle as a launch of its own (k_begin_cycle)
+   static void begin(const DevState &s, hipStream_t st);
+   // end of a device loop (k_run_end)
+   static void run_end(const DevState &s, double *slots0, int32_t *err0, hipStream_t st);
 };
 
 extern template struct Launch<PolicyFp64>;

@@ -8,10 +8,11 @@
 
 namespace lgpu {
 
-// TimeIncrement operands plus the loop flag the kernels test.
+// TimeIncrement operands plus the loop flag the kernels test.  fresh: no cycle
+// of this loop has run, so dtcourant and dthydro are the caller's.
 struct DevTime {
    double time, deltatime, dtcourant, dthydro, stoptime, dtfixed, dtmax, multlb, multub;
-   int32_t cycle, maxCycle, active, pad;
+   int32_t cycle, maxCycle, active, fresh;
 };
 
 // TimeIncrement (lulesh.cc:166-222) at the top of a cycle, given the dt
