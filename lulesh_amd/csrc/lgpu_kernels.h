@@ -83,6 +83,11 @@ struct PolicyFp64 {
    // waves per SIMD (min, max) for the nodal brick kernel's register
    // allocation and scheduling; (1, 8) leaves it to the compiler
    static constexpr int kNodalWavesMin = 1, kNodalWavesMax = 8;
+   // the ensemble form takes a register or two more for its members' tiles, and
+   // FP64_FMA then has 258, for one wave per SIMD: held to two waves, 64 members
+   // of 16..64 602 -> 470 us.  The single problem's form has 256 by itself
+   // (held to them it spills 3, s=96 63.9 -> 64.9 us)
+   static constexpr int kMemberWavesMin = 2;
    // brick kernel: load the node update's operands before the element work
    static constexpr bool kPrefetchNode = true;
    // brick kernel: 32-bit byte offsets from scalar bases (at32) instead of
@@ -135,6 +140,7 @@ struct PolicyMixed {
    // exactly 3: aiming for 4 (128 VGPRs) makes the scheduler issue the
    // hourglass velocity loads one at a time, each waited on at once
    static constexpr int kNodalWavesMin = 3, kNodalWavesMax = 3;
+   static constexpr int kMemberWavesMin = 3;
    static constexpr bool kPrefetchNode = true;
    static constexpr bool kOffset32 = true;
    static constexpr bool kHgVelEarly = true;
