@@ -210,10 +210,13 @@ struct EnsTime {
    int32_t *maxCycle;
 };
 
-// Results of a cycle in pinned host memory, for lgpu_time_constraints.
+// What the host polls, in pinned host memory: results of k_dt_slots or
+// k_run_end, with the launch's count seq stored after them, and of a device
+// loop the count of the last cycle begun and whether the loop has ended.
 struct HostOut {
    double dt[2];
    int32_t err[kNumErrSites];
+   uint32_t seq, started, ended;
 };
 
 // Everything a cycle touches on the device.
@@ -258,7 +261,8 @@ struct DevState {
    struct DevTime *timeOut;
    const int32_t *errPrev;
    double *dtPartialPrev;
-   HostOut *hostOut;        // one problem, host-driven: the results again (or null)
+   HostOut *hostOut;        // one problem (null: ensembles)
+   uint32_t hostSeq;        // what this launch stores in hostOut->seq or started
    const double *dtDevice;  // device-side deltatime (null: use argument)
    const int32_t *active;   // device-side loop flag (null: always active)
    Brick brick;             // valid when isBrick

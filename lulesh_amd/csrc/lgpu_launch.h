@@ -10,6 +10,7 @@
 #include <vector>
 
 #include "lgpu_kernels.h"
+#include "lgpu_time.h"
 
 namespace lgpu {
 
@@ -85,8 +86,10 @@ struct Launch {
    static void dt_reduce(const DevState &s, hipStream_t st);
    // start of a device-loop cycle as a launch of its own (k_begin_cycle)
    static void begin(const DevState &s, hipStream_t st);
-   // end of a device loop (k_run_end)
-   static void run_end(const DevState &s, double *slots0, int32_t *err0, hipStream_t st);
+   // start and end of a device loop (k_run_start, k_run_end)
+   static void run_start(const DevTime &t, DevTime *time, double *dtOut, hipStream_t st);
+   static void run_end(const DevState &s, double *slots0, int32_t *err0, DevTime *hostTime,
+                       hipStream_t st);
 };
 
 extern template struct Launch<PolicyFp64>;

@@ -20,6 +20,8 @@ def _context(o, form):
     ctx = context_from_oracle(o, generic=form == "generic")
     if form == "walk":  # the cycle start is a launch
         ctx.set_option(la.native.OPT_BRICK_CHUNK, 3)
+    if form == "timed":  # waits for the stream instead of the kernels' counts
+        ctx.set_option(la.native.OPT_KERNEL_TIMING, 1)
     upload_state(ctx, o)
     return ctx
 
@@ -32,12 +34,12 @@ def _time_state(o):
     return ts
 
 
-@pytest.mark.parametrize("form", ["block", "walk", "generic"])
+@pytest.mark.parametrize("form", ["block", "walk", "generic", "timed"])
 def test_runs_in_pieces_match_the_oracle(form):
     o = OracleDomain(7, 3, 1, 1)
     ctx = _context(o, form)
     ts = _time_state(o)
-    for its in (1, 1, 2, 0, 3, 16, 17, 33):  # odd, even, around a batch of 16
+    for its in (1, 1, 2, 0, 3, 16, 17, 33):  # odd, even, around the 16 that the host runs ahead
         assert o.run(ts.cycle + its) == 0  # both take the last cycle
         assert ctx.run(ts, ts.cycle + its) == 0
         for f in TIMES:  # FP64 keeps the oracle's rounding
