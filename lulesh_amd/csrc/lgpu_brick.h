@@ -4,6 +4,7 @@
 #pragma once
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <cstdint>
 #include <vector>
@@ -92,24 +93,60 @@ inline void set_brick_chunk(Brick &g, int chunk)
    g.chunks = (g.en + g.chunkZ - 1) / g.chunkZ;
 }
 
-// Time of a column-walking launch in planes: `columns` column tiles, each cut
-// into z-chunks of `chunk` planes out of `planes`, run in rounds of `slots`
-// resident workgroups, and a workgroup walks one plane more than its chunk.
-inline int64_t walk_cost(int64_t columns, int planes, int slots, int chunk)
+// A column-walking launch: `columns` column tiles, each cut into z-chunks of
+// `chunk` planes out of `planes` and, where that does not come out even, a
+// shorter last one, on `slots` resident workgroups.  A walk takes its planes
+// and `extra` of one more.  The whole chunks are dispatched first and the
+// last ones (logical_block's second part) into the slots that these leave.
+struct WalkTime {
+   double whole; // end of the whole chunks, in planes
+   double end;   // end of the launch
+   double work;  // planes walked per slot
+};
+
+inline WalkTime walk_time(int64_t columns, int planes, int slots, int chunk, double extra)
 {
-   const int64_t blocks = columns * ((planes + chunk - 1) / chunk);
-   return (blocks + slots - 1) / slots * (chunk + 1);
+   const int64_t wholes = columns * (planes / chunk), last = planes % chunk ? columns : 0;
+   const double walk = chunk + extra, lastWalk = planes % chunk + extra;
+   const int64_t rounds = wholes / slots, left = wholes % slots, open = slots - left;
+   WalkTime t;
+   t.whole = t.end = walk * (double)(rounds + (left ? 1 : 0));
+   t.work = ((double)wholes * walk + (double)last * lastWalk) / slots;
+   if (last) {
+      // back to back in the slots that the last round of whole chunks leaves
+      // open, begun while that round lasts, and in all of them after it
+      const int64_t turns = left ? (int64_t)std::ceil(walk / lastWalk) : last;
+      const int64_t early = std::min(last, turns * open), late = last - early;
+      t.end = std::max({t.whole, walk * (double)rounds + lastWalk * (double)((early + open - 1) / open),
+                        t.whole + lastWalk * (double)((late + slots - 1) / slots)});
+   }
+   return t;
 }
 
-// The chunk (at least `least` planes) with the smallest walk_cost: redundant
-// planes against a partly filled last round.
-inline int pick_chunk(int64_t columns, int planes, int slots, int least, int fallback)
+// Time of the fused nodal kernel's walk in planes.  The last chunks that run
+// beyond the others have a CU's units to themselves and count half.  FP64,
+// chunk by rounds of equal chunks / by this, us: s=90 10 / 9, 82 / 75; s=101
+// 11 / 10, 88 / 82; s=128 22 / 21, 180 / 173; s=160 41 / 39, 327 / 311; s=192
+// 65 / 64, 511 / 505; s=200 41 / 39, 635 / 611.
+inline double walk_cost(int64_t columns, int planes, int slots, int chunk)
 {
-   if (slots < 1) return fallback;
-   int best = fallback;
-   int64_t bestCost = INT64_MAX;
-   for (int ch = least; ch <= planes; ++ch) {
-      const int64_t cost = walk_cost(columns, planes, slots, ch);
+   const WalkTime t = walk_time(columns, planes, slots, chunk, 1.0);
+   return 0.5 * (t.whole + t.end);
+}
+
+// Default node planes per workgroup of the fused nodal kernel (at least
+// `least`): the smallest walk_cost, redundant planes against idle slots.  Long
+// walks drift apart and lose their neighbours' planes in L2, so more than 40
+// planes are walked only in a single round, and never more than 66: FP64 s=210
+// chunk 94 759 us, 47 777, 23 714; s=220 99 800, 49 816, 24 751.
+inline int pick_brick_chunk(const Brick &g, int slots, int least)
+{
+   int best = 8;
+   double bestCost = 1e300;
+   const int64_t columns = (int64_t)g.tilesX * g.tilesY;
+   for (int ch = least; slots > 0 && ch <= std::min(g.en, 66); ++ch) {
+      if (ch > 40 && columns * (g.en / ch) > slots) continue;
+      const double cost = walk_cost(columns, g.en, slots, ch);
       if (cost < bestCost) {
          bestCost = cost;
          best = ch;
@@ -118,20 +155,12 @@ inline int pick_chunk(int64_t columns, int planes, int slots, int least, int fal
    return best;
 }
 
-// Default node planes per workgroup of the fused nodal kernel.  s=192 on
-// 256 CUs: 65 for FP64 (2 workgroups per CU: all 507 resident at once, 2%
-// faster than 22), 22 for the mixed form (3 per CU).
-inline int pick_brick_chunk(const Brick &g, int slots, int least)
-{
-   return pick_chunk((int64_t)g.tilesX * g.tilesY, g.en, slots, least, 8);
-}
-
 // The chunk for launches of several rounds whose workgroups end at different
 // times (the mixed form, 3 a CU; ensembles, whose members' last chunks are
 // shorter): least work per resident workgroup, plus half a walk for the tail
-// of the launch.  columns[i] column tiles of planes[i] planes each.  Mixed:
-// s=192 chunk 22 -> 13, 412 -> 401 us; s=160 22 -> 7, 276 -> 242; s=128 15 ->
-// 5, 138 -> 133 (fewest rounds against this).
+// of the launch.  columns[i] column tiles of planes[i] planes each.  Fewest
+// rounds / this, mixed: s=192 chunk 22 / 9, 405 / 395 us; s=160 22 / 7, 276 /
+// 241; s=128 14 / 5, 129 / 125.
 inline int pick_tail_chunk(const std::vector<int64_t> &columns, const std::vector<int> &planes,
                            int slots, int fallback)
 {
@@ -157,12 +186,26 @@ inline void set_kin_chunk(Brick &g, int chunk)
    g.kinChunks = (g.s + g.kinChunk - 1) / g.kinChunk;
 }
 
-// Default element planes per workgroup of the kinematics kernel.  s=192 on
-// 256 CUs: 12 for FP64 (3 workgroups per CU), 28 for the mixed form (4 per
-// CU: 1,008 workgroups, all resident at once; 3% faster than 12).
+// Default element planes per workgroup of the kinematics kernel: 4 to 12 (long
+// walks drift apart and lose their neighbours' planes in L2), by the end of
+// the launch, the work per slot and a fifth of a walk.  Its extra plane is
+// only copied, which counts as 0.3.  By rounds of equal chunks / by this, us,
+// FP64: s=160 7 / 7, 124 / 123; s=175 30 / 7, 185 / 168; s=185 37 / 7, 221 / 207;
+// s=192 12 / 12, 200 / 200; s=200 23 / 9, 255 / 250; s=220 20 / 7, 361 / 338;
+// mixed s=175 30 / 7, 155 / 132; s=192 12 / 9, 154 / 155.
 inline int pick_kin_chunk(const Brick &g, int slots)
 {
-   return pick_chunk((int64_t)g.kinTiles * g.kinTiles, g.s, slots, 4, 12);
+   int best = 12;
+   double bestCost = 1e300;
+   for (int ch = 4; slots > 0 && ch <= std::min(12, g.s); ++ch) {
+      const WalkTime t = walk_time((int64_t)g.kinTiles * g.kinTiles, g.s, slots, ch, 0.3);
+      const double cost = t.end + t.work + 0.2 * (ch + 0.3);
+      if (cost < bestCost) {
+         bestCost = cost;
+         best = ch;
+      }
+   }
+   return best;
 }
 
 // Fused nodal kernel tiles of w threads by h rows: (w-1) x (h-1) nodes each.
@@ -261,9 +304,9 @@ inline int64_t block_blocks(const Brick &g) { return (int64_t)g.blkX * g.blkY * 
 // 21.1 / 41.5, s=60 34.4 / 41.4, s=76 53.8 / 55.7; walk taken: s=59 31.5 /
 // 27.8, s=74 55.1 / 42.5, s=101 119.8 / 92.3.  FP64_FMA s=64 33.9 / 35.0,
 // mixed s=30 9.8 / 13.7, s=63 25.0 / 26.7.
-inline bool block_is_faster(int64_t blocks, int slots, int64_t cost)
+inline bool block_is_faster(int64_t blocks, int slots, double cost)
 {
-   return slots > 0 && 5 * blocks < (5 * cost - 3) * slots;
+   return slots > 0 && (double)blocks < (cost - 0.6) * slots;
 }
 
 // The largest brick of k_kin_flat.  Flat / best walk: FP64 s=30 8.5 / 9.0 us

@@ -276,11 +276,11 @@ void pick_brick_kernels(lgpu_ensemble *e)
       planes.push_back(g.en);
    }
    e->nodalChunk = pick_tail_chunk(columns, planes, slots, e->nodalChunk);
-   int64_t least = INT64_MAX;
+   double least = 1e300;
    for (int ch = 1; ch <= 22; ++ch) {
       int64_t walks = 0;
       for (const Brick &g : bricks) walks += (int64_t)g.tilesX * g.tilesY * ((g.en + ch - 1) / ch);
-      least = std::min(least, (walks + slots - 1) / slots * (ch + 1));
+      least = std::min(least, (double)((walks + slots - 1) / slots * (ch + 1)));
    }
    e->s.nodalBlock = block_is_faster(blocks, slots, least);
 }
