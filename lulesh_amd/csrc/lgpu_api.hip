@@ -516,7 +516,7 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
       if (s.nodalBlock) // the chunk the walk would start from, should an option select it
          set_brick_chunk(g, pick_brick_chunk(g, slots, 4));
       else if (sp.precision == LGPU_MIXED)
-         set_brick_chunk(g, pick_tail_chunk({(int64_t)g.tilesX * g.tilesY}, {g.en}, slots, g.chunkZ));
+         set_brick_chunk(g, pick_tail_chunk({(int64_t)g.tilesX * g.tilesY}, {g.en}, slots, 0.5, g.chunkZ));
       s.kinFlat = g.s <= kKinFlatMax;
       int kinPerCu = 0;
       switch (sp.precision) {

@@ -156,13 +156,15 @@ inline int pick_brick_chunk(const Brick &g, int slots, int least)
 }
 
 // The chunk for launches of several rounds whose workgroups end at different
-// times (the mixed form, 3 a CU; ensembles, whose members' last chunks are
-// shorter): least work per resident workgroup, plus half a walk for the tail
-// of the launch.  columns[i] column tiles of planes[i] planes each.  Fewest
-// rounds / this, mixed: s=192 chunk 22 / 9, 405 / 395 us; s=160 22 / 7, 276 /
-// 241; s=128 14 / 5, 129 / 125.
+// times (the mixed form, 3 a CU; ensembles): least work per resident workgroup,
+// plus a part of a walk for the end of the launch, a quarter in an ensemble,
+// whose many short last chunks fill it.  columns[i] column tiles of planes[i]
+// planes each.  Fewest rounds / this, mixed: s=192 chunk 22 / 9, 405 / 395 us;
+// s=160 22 / 7, 276 / 241; s=128 14 / 5, 129 / 125.  Half / quarter, FP64: 64
+// members of 16..64 11 / 16, 486 / 482; 30 of 10..40 5 / 7, 98 / 92; 16 of 40..90
+// 12 / 18, 530 / 529; mixed 40 of 20..50 6 / 8, 164 / 159.
 inline int pick_tail_chunk(const std::vector<int64_t> &columns, const std::vector<int> &planes,
-                           int slots, int fallback)
+                           int slots, double part, int fallback)
 {
    if (slots < 1) return fallback;
    int best = fallback;
@@ -171,7 +173,7 @@ inline int pick_tail_chunk(const std::vector<int64_t> &columns, const std::vecto
       double walked = 0.;
       for (size_t i = 0; i < columns.size(); ++i)
          walked += (double)columns[i] * (planes[i] + (planes[i] + ch - 1) / ch);
-      const double work = std::max(walked / slots + 0.5 * (ch + 1), ch + 1.0);
+      const double work = std::max(walked / slots + part * (ch + 1), ch + 1.0);
       if (work < bestWork) {
          bestWork = work;
          best = ch;
@@ -337,9 +339,5 @@ inline void init_brick(Brick &g, int s)
    set_kin_chunk(g, 12);
    pick_nodal_block(g);
 }
-
-// Workgroups of one launch of each brick kernel.
-inline int64_t nodal_blocks(const Brick &g) { return (int64_t)g.tilesX * g.tilesY * g.chunks; }
-inline int64_t kin_blocks(const Brick &g) { return (int64_t)g.kinTilesX * g.kinTilesY * g.kinChunks; }
 
 } // namespace lgpu

@@ -241,10 +241,9 @@ int launch_graph(lgpu_ensemble *e)
 }
 
 // The brick path's default kernels and nodal chunk.  A walk's cost is taken
-// over all members' workgroups.  64
-// members of 16..64, FP64: chunk 10, 500 us (7: 495, 4: 519); 30 of 10..40:
-// chunk 4, 68.7 us (8: 81.8, k_nodal_block 84.8); 24 of 5..24: k_nodal_block,
-// FP64 18.6 and mixed 13.6 us (best walk 24.1 and 18.5).
+// over all members' workgroups.  30 members of 10..40: a walk, 68.7 us
+// (k_nodal_block 84.8); 24 of 5..24: k_nodal_block, FP64 18.6 and mixed 13.6
+// us (best walk 24.1 and 18.5).
 void pick_brick_kernels(lgpu_ensemble *e)
 {
    int dev = 0, cus = 0, perCu = 0, largest = 0;
@@ -275,7 +274,7 @@ void pick_brick_kernels(lgpu_ensemble *e)
       columns.push_back((int64_t)g.tilesX * g.tilesY);
       planes.push_back(g.en);
    }
-   e->nodalChunk = pick_tail_chunk(columns, planes, slots, e->nodalChunk);
+   e->nodalChunk = pick_tail_chunk(columns, planes, slots, 0.25, e->nodalChunk);
    double least = 1e300;
    for (int ch = 1; ch <= 22; ++ch) {
       int64_t walks = 0;
@@ -285,14 +284,46 @@ void pick_brick_kernels(lgpu_ensemble *e)
    e->s.nodalBlock = block_is_faster(blocks, slots, least);
 }
 
-// Member tables of the brick path for the current kernel and chunk choices: per-member
-// bricks with offsets and first workgroups, and workgroup -> member maps.
+// The workgroups of a walking kernel over all members: those of whole z-chunks
+// by member, then the members' last, shorter chunks, longest first, so that
+// the launch does not end on a long walk.  Members: `columns` column tiles of
+// `planes` planes each; returns the number of the first.  64 members of
+// 16..64, FP64 nodal, by member throughout / so: chunk 10 522 / 485 us, 16 531 /
+// 482; mixed chunk 9 399 / 378.
+int32_t walk_blocks(const std::vector<int64_t> &columns, const std::vector<int> &planes, int chunk,
+                    std::vector<MemberBlock> &blocks)
+{
+   std::vector<std::vector<MemberBlock>> last((size_t)chunk); // by length
+   for (size_t m = 0; m < columns.size(); ++m) {
+      const uint32_t n = (uint32_t)(columns[m] * (planes[m] / chunk));
+      for (uint32_t w = 0; w < n; ++w) blocks.push_back(MemberBlock{(int32_t)m, w});
+      const int rest = planes[m] % chunk;
+      for (uint32_t w = 0; rest && w < (uint32_t)columns[m]; ++w)
+         last[(size_t)rest].push_back(MemberBlock{(int32_t)m, n + w});
+   }
+   const int32_t whole = (int32_t)blocks.size();
+   for (int rest = chunk - 1; rest > 0; --rest)
+      blocks.insert(blocks.end(), last[(size_t)rest].begin(), last[(size_t)rest].end());
+   return whole;
+}
+
+// The same for kernels of equal workgroups, blocks[m] of member m.
+int32_t equal_blocks(const std::vector<int64_t> &counts, std::vector<MemberBlock> &blocks)
+{
+   for (size_t m = 0; m < counts.size(); ++m)
+      for (uint32_t w = 0; w < (uint32_t)counts[m]; ++w) blocks.push_back(MemberBlock{(int32_t)m, w});
+   return (int32_t)blocks.size();
+}
+
+// Member tables of the brick path for the current kernel and chunk choices:
+// per-member bricks with offsets, and the kernels' workgroups.
 int build_brick_tables(lgpu_ensemble *e)
 {
    const int M = e->nMembers;
    std::vector<MemberBrick> mb((size_t)M);
-   std::vector<int32_t> nodalOf, kinOf;
-   int64_t nb = 0, kb = 0;
+   std::vector<MemberBlock> nodal, kin;
+   std::vector<int64_t> nodalCount, kinCount; // workgroups, or column tiles of the walks
+   std::vector<int> nodePlanes, elemPlanes;
    for (int m = 0; m < M; ++m) {
       Brick g{};
       init_brick(g, e->memberSize[(size_t)m]);
@@ -303,17 +334,18 @@ int build_brick_tables(lgpu_ensemble *e)
       mb[(size_t)m].g = g;
       mb[(size_t)m].nodeOff = e->nodeStart[(size_t)m];
       mb[(size_t)m].elemOff = e->elemStart[(size_t)m];
-      mb[(size_t)m].nodalBlock0 = (int32_t)nb;
-      mb[(size_t)m].kinBlock0 = (int32_t)kb;
-      const int64_t n1 = e->s.nodalBlock ? block_blocks(g) : nodal_blocks(g);
-      const int64_t k1 = e->s.kinFlat ? flat_blocks(g) : kin_blocks(g);
-      nodalOf.insert(nodalOf.end(), (size_t)n1, m);
-      kinOf.insert(kinOf.end(), (size_t)k1, m);
-      nb += n1;
-      kb += k1;
+      nodalCount.push_back(e->s.nodalBlock ? block_blocks(g) : (int64_t)g.tilesX * g.tilesY);
+      kinCount.push_back(e->s.kinFlat ? flat_blocks(g) : (int64_t)g.kinTilesX * g.kinTilesY);
+      nodePlanes.push_back(g.en);
+      elemPlanes.push_back(g.s);
    }
+   e->s.nodalWhole = e->s.nodalBlock ? equal_blocks(nodalCount, nodal)
+                                     : walk_blocks(nodalCount, nodePlanes, e->nodalChunk, nodal);
+   e->s.kinWhole = e->s.kinFlat ? equal_blocks(kinCount, kin)
+                                : walk_blocks(kinCount, elemPlanes, e->kinChunk, kin);
+   const size_t nb = nodal.size(), kb = kin.size();
    const size_t b0 = align_up(sizeof(MemberBrick) * (size_t)M);
-   const size_t b1 = align_up(4 * (size_t)nb), b2 = align_up(4 * (size_t)kb);
+   const size_t b1 = align_up(sizeof(MemberBlock) * nb), b2 = align_up(sizeof(MemberBlock) * kb);
    const size_t need = b0 + b1 + b2;
    ENS_HIP(e, hipStreamSynchronize(e->stream));
    if (need > e->tablesBytes) {
@@ -324,11 +356,11 @@ int build_brick_tables(lgpu_ensemble *e)
       e->tablesBytes = need;
    }
    ENS_HIP(e, hipMemcpy(e->tables, mb.data(), sizeof(MemberBrick) * (size_t)M, hipMemcpyHostToDevice));
-   ENS_HIP(e, hipMemcpy(e->tables + b0, nodalOf.data(), 4 * (size_t)nb, hipMemcpyHostToDevice));
-   ENS_HIP(e, hipMemcpy(e->tables + b0 + b1, kinOf.data(), 4 * (size_t)kb, hipMemcpyHostToDevice));
+   ENS_HIP(e, hipMemcpy(e->tables + b0, nodal.data(), sizeof(MemberBlock) * nb, hipMemcpyHostToDevice));
+   ENS_HIP(e, hipMemcpy(e->tables + b0 + b1, kin.data(), sizeof(MemberBlock) * kb, hipMemcpyHostToDevice));
    e->s.memberBrick = reinterpret_cast<const MemberBrick *>(e->tables);
-   e->s.nodalBlockMember = reinterpret_cast<const int32_t *>(e->tables + b0);
-   e->s.kinBlockMember = reinterpret_cast<const int32_t *>(e->tables + b0 + b1);
+   e->s.nodalBlocks = reinterpret_cast<const MemberBlock *>(e->tables + b0);
+   e->s.kinBlocks = reinterpret_cast<const MemberBlock *>(e->tables + b0 + b1);
    e->nodalBlocks = (unsigned)nb;
    e->kinBlocks = (unsigned)kb;
    drop_graph(e);

@@ -193,11 +193,16 @@ struct Brick {
 };
 
 // One ensemble member on the brick path: its brick, where its nodes and
-// elements start in the concatenated arrays, and its first workgroup in the
-// k_nodal_brick and k_kin_brick grids.
+// elements start in the concatenated arrays.
 struct MemberBrick {
    Brick g;
-   int32_t nodeOff, elemOff, nodalBlock0, kinBlock0;
+   int32_t nodeOff, elemOff;
+};
+
+// One workgroup of a brick kernel in an ensemble.
+struct MemberBlock {
+   int32_t member;
+   uint32_t wg; // within the member's grid
 };
 
 // Per-member time state of an ensemble, struct of arrays (the kernels read
@@ -284,8 +289,11 @@ struct DevState {
    EnsTime ensTime;                // the members' next TimeIncrement
    // ensemble on the brick path (memberBrick non-null)
    const MemberBrick *memberBrick;
-   const int32_t *nodalBlockMember; // k_nodal_brick workgroup -> member
-   const int32_t *kinBlockMember;   // k_kin_brick workgroup -> member
+   const MemberBlock *nodalBlocks; // the nodal brick kernels' workgroups
+   const MemberBlock *kinBlocks;   // the kinematics brick kernels' workgroups
+   // the first ones, whole chunks, are mapped to XCDs; those after them are
+   // shorter and dealt out longest first
+   int32_t nodalWhole, kinWhole;
 };
 
 } // namespace lgpu
