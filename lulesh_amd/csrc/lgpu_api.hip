@@ -7,7 +7,6 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <chrono>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -22,6 +21,7 @@
 #include "lgpu_launch.h"
 #include "lgpu_setup.h"
 #include "lgpu_time.h"
+#include "lgpu_wait.h"
 #include "lulesh_gpu.h"
 
 using namespace lgpu;
@@ -71,11 +71,12 @@ struct lgpu_ctx {
    size_t arenaBytes = 0;
    int64_t planeStride = 0; // corner plane length (elements, padded)
    DevState s{};
-   // pinned readback: dt[2], err[kNumErrSites]
+   // pinned: HostOut (dt[2], err[kNumErrSites], counts), time state, SmallCopy
    double *hostDt = nullptr;
    int32_t *hostErr = nullptr;
    bool hostOutFresh = false; // the last launch leaves its results in s.hostOut
    uint32_t hostSeq = 0, cycleSeq = 0; // last seq and started of s.hostOut asked for
+   SmallCopy small;
    DevTime *devTime = nullptr;
    DevTime *hostTime = nullptr;
    // diagnostics storage (allocated on first use)
@@ -116,22 +117,6 @@ hipEvent_t take_event(lgpu_ctx *c)
 
 // Folds finished timed launches into the per-kernel totals.  Call only after
 // the stream has been synchronized.
-// Waits until a kernel's count in pinned memory has reached `want`, for up to
-// 2 ms: false if it has not, and the caller then waits for the stream.  A
-// kernel's store is seen about 5 us sooner than hipStreamSynchronize returns
-// (launch and wait 5.8 against 11.3 us), of no weight after 2 ms.
-bool host_reached(const uint32_t *count, uint32_t want)
-{
-   const auto start = std::chrono::steady_clock::now();
-   for (;;) {
-      for (int i = 0; i < 64; ++i) {
-         if ((int32_t)(__atomic_load_n(count, __ATOMIC_ACQUIRE) - want) >= 0) return true;
-         __builtin_ia32_pause();
-      }
-      if (std::chrono::steady_clock::now() - start > std::chrono::milliseconds(2)) return false;
-   }
-}
-
 void harvest_timing(lgpu_ctx *c)
 {
    for (TimedLaunch &t : c->pending) {
@@ -573,13 +558,15 @@ int finish_context(lgpu_ctx *c)
    const int st = set_eos_order(c, 4);
    if (st != LGPU_OK) return st;
    if (hipHostMalloc((void **)&c->hostDt, sizeof(double) * 2 + sizeof(int32_t) * kNumErrSites +
-                                               sizeof(DevTime) + 64, hipHostMallocDefault) != hipSuccess)
+                                               sizeof(DevTime) + 64 + kSmallCopyBytes,
+                     hipHostMallocDefault) != hipSuccess)
       return LGPU_ENOMEM;
    c->hostErr = reinterpret_cast<int32_t *>(c->hostDt + 2);
    static_assert(sizeof(HostOut) <= 64, "hostTime follows at 64 bytes");
    c->s.hostOut = reinterpret_cast<HostOut *>(c->hostDt);
    *c->s.hostOut = HostOut{};
    c->hostTime = reinterpret_cast<DevTime *>(reinterpret_cast<char *>(c->hostDt) + 64);
+   c->small.init(c->hostTime + 1);
    return LGPU_OK;
 }
 
@@ -877,6 +864,10 @@ int lgpu_upload(lgpu_ctx *c, int field, const double *host)
    double *dst = real_field_ptr(c, field, isElem, narrow);
    if (!dst) return LGPU_EINVAL;
    const size_t n = isElem ? (size_t)c->numElem : (size_t)c->numNode;
+   if ((int64_t)n <= kSmallCopy) {
+      HIP_OR_RETURN(c, c->small.upload(host, dst, narrow, (int)n, c->stream));
+      return LGPU_OK;
+   }
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
    if (narrow && (int64_t)n > kConvertOnHost) {
       double *wide = scratch_doubles(c);
@@ -899,6 +890,10 @@ int lgpu_download(lgpu_ctx *c, int field, double *host)
    bool isElem, narrow;
    double *src = real_field_ptr(c, field, isElem, narrow);
    const size_t n = isElem ? (size_t)c->numElem : (size_t)c->numNode;
+   if (src && (int64_t)n <= kSmallCopy) {
+      HIP_OR_RETURN(c, c->small.download(src, host, narrow, (int)n, c->stream));
+      return LGPU_OK;
+   }
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
    if (!src) {
       std::fill(host, host + n, 0.0);

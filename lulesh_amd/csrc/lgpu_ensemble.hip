@@ -82,8 +82,9 @@ struct lgpu_ensemble {
    int64_t kLaunches[kENumKernels] = {};
    double kMs[kENumKernels] = {};
    std::string lastError;
-   // pinned host mirror of the time state
+   // pinned: SmallCopy, host mirror of the time state
    char *host = nullptr;
+   SmallCopy small;
 };
 
 namespace {
@@ -663,10 +664,11 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    if (!ok) return bail(LGPU_EDEVICE);
    if (e->brick) pick_brick_kernels(e);
    if (e->brick && build_brick_tables(e) != LGPU_OK) return bail(LGPU_EDEVICE);
-   if (hipHostMalloc((void **)&e->host, (size_t)nMembers * (9 * 8 + 8) + 64 +
+   if (hipHostMalloc((void **)&e->host, kSmallCopyBytes + (size_t)nMembers * (9 * 8 + 8) + 64 +
                                             (size_t)nMembers * kNumErrSites * 4,
                      hipHostMallocDefault) != hipSuccess)
       return bail(LGPU_ENOMEM);
+   e->small.init(e->host);
    *out = e;
    return LGPU_OK;
 }
@@ -691,18 +693,23 @@ int lgpu_ensemble_upload(lgpu_ensemble *e, int32_t member, int field, const doub
    if (!base) return LGPU_EINVAL;
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
+   void *dst = narrow ? (void *)(reinterpret_cast<float *>(base) + off) : (void *)(base + off);
+   if ((int64_t)n <= kSmallCopy) {
+      ENS_HIP(e, e->small.upload(host, dst, narrow, (int)n, e->stream));
+      return LGPU_OK;
+   }
    ENS_HIP(e, hipStreamSynchronize(e->stream));
    if (narrow && (int64_t)n > kConvertOnHost) {
       double *wide = scratch_doubles(e);
       ENS_HIP(e, hipMemcpy(wide, host, 8 * n, hipMemcpyHostToDevice));
-      ENS_HIP(e, launch_narrow(wide, reinterpret_cast<float *>(base) + off, (int64_t)n, e->stream));
+      ENS_HIP(e, launch_narrow(wide, static_cast<float *>(dst), (int64_t)n, e->stream));
       ENS_HIP(e, hipStreamSynchronize(e->stream));
    } else if (narrow) {
       std::vector<float> tmp(n);
       for (size_t i = 0; i < n; ++i) tmp[i] = (float)host[i];
-      ENS_HIP(e, hipMemcpy(reinterpret_cast<float *>(base) + off, tmp.data(), 4 * n, hipMemcpyHostToDevice));
+      ENS_HIP(e, hipMemcpy(dst, tmp.data(), 4 * n, hipMemcpyHostToDevice));
    } else {
-      ENS_HIP(e, hipMemcpy(base + off, host, 8 * n, hipMemcpyHostToDevice));
+      ENS_HIP(e, hipMemcpy(dst, host, 8 * n, hipMemcpyHostToDevice));
    }
    return LGPU_OK;
 }
@@ -715,18 +722,23 @@ int lgpu_ensemble_download(lgpu_ensemble *e, int32_t member, int field, double *
    if (!base) return LGPU_EINVAL;
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
+   const void *src = narrow ? (const void *)(reinterpret_cast<float *>(base) + off) : (const void *)(base + off);
+   if ((int64_t)n <= kSmallCopy) {
+      ENS_HIP(e, e->small.download(src, host, narrow, (int)n, e->stream));
+      return LGPU_OK;
+   }
    ENS_HIP(e, hipStreamSynchronize(e->stream));
    if (narrow && (int64_t)n > kConvertOnHost) {
       double *wide = scratch_doubles(e);
-      ENS_HIP(e, launch_widen(reinterpret_cast<const float *>(base) + off, wide, (int64_t)n, e->stream));
+      ENS_HIP(e, launch_widen(static_cast<const float *>(src), wide, (int64_t)n, e->stream));
       ENS_HIP(e, hipStreamSynchronize(e->stream));
       ENS_HIP(e, hipMemcpy(host, wide, 8 * n, hipMemcpyDeviceToHost));
    } else if (narrow) {
       std::vector<float> tmp(n);
-      ENS_HIP(e, hipMemcpy(tmp.data(), reinterpret_cast<float *>(base) + off, 4 * n, hipMemcpyDeviceToHost));
+      ENS_HIP(e, hipMemcpy(tmp.data(), src, 4 * n, hipMemcpyDeviceToHost));
       for (size_t i = 0; i < n; ++i) host[i] = tmp[i];
    } else {
-      ENS_HIP(e, hipMemcpy(host, base + off, 8 * n, hipMemcpyDeviceToHost));
+      ENS_HIP(e, hipMemcpy(host, src, 8 * n, hipMemcpyDeviceToHost));
    }
    return LGPU_OK;
 }
@@ -736,7 +748,7 @@ int lgpu_ensemble_run(lgpu_ensemble *e, lgpu_time_state *ts, int32_t maxCycle, i
    if (!e || !ts) return LGPU_EINVAL;
    const int M = e->nMembers;
    // Pinned staging: 9 double arrays, cycle, active, err.
-   double *hd = reinterpret_cast<double *>(e->host);
+   double *hd = reinterpret_cast<double *>(e->host + kSmallCopyBytes);
    int32_t *hcyc = reinterpret_cast<int32_t *>(hd + 9 * (size_t)M);
    int32_t *hact = hcyc + M;
    int32_t *herr = hact + M;
