@@ -557,16 +557,16 @@ int finish_context(lgpu_ctx *c)
    // regions).
    const int st = set_eos_order(c, 4);
    if (st != LGPU_OK) return st;
-   if (hipHostMalloc((void **)&c->hostDt, sizeof(double) * 2 + sizeof(int32_t) * kNumErrSites +
-                                               sizeof(DevTime) + 64 + kSmallCopyBytes,
-                     hipHostMallocDefault) != hipSuccess)
+   constexpr size_t kSmallAt = (64 + sizeof(DevTime) + 63) / 64 * 64;
+   if (hipHostMalloc((void **)&c->hostDt, kSmallAt + small_copy_bytes(kSmallNarrow), hipHostMallocDefault) !=
+       hipSuccess)
       return LGPU_ENOMEM;
    c->hostErr = reinterpret_cast<int32_t *>(c->hostDt + 2);
    static_assert(sizeof(HostOut) <= 64, "hostTime follows at 64 bytes");
    c->s.hostOut = reinterpret_cast<HostOut *>(c->hostDt);
    *c->s.hostOut = HostOut{};
    c->hostTime = reinterpret_cast<DevTime *>(reinterpret_cast<char *>(c->hostDt) + 64);
-   c->small.init(c->hostTime + 1);
+   c->small.init(reinterpret_cast<char *>(c->hostDt) + kSmallAt);
    return LGPU_OK;
 }
 
@@ -864,7 +864,7 @@ int lgpu_upload(lgpu_ctx *c, int field, const double *host)
    double *dst = real_field_ptr(c, field, isElem, narrow);
    if (!dst) return LGPU_EINVAL;
    const size_t n = isElem ? (size_t)c->numElem : (size_t)c->numNode;
-   if ((int64_t)n <= kSmallCopy) {
+   if (c->small.takes(n, narrow)) {
       HIP_OR_RETURN(c, c->small.upload(host, dst, narrow, (int)n, c->stream));
       return LGPU_OK;
    }
@@ -890,7 +890,7 @@ int lgpu_download(lgpu_ctx *c, int field, double *host)
    bool isElem, narrow;
    double *src = real_field_ptr(c, field, isElem, narrow);
    const size_t n = isElem ? (size_t)c->numElem : (size_t)c->numNode;
-   if (src && (int64_t)n <= kSmallCopy) {
+   if (src && c->small.takes(n, narrow)) {
       HIP_OR_RETURN(c, c->small.download(src, host, narrow, (int)n, c->stream));
       return LGPU_OK;
    }

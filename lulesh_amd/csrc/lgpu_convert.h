@@ -17,26 +17,33 @@ constexpr int64_t kConvertOnHost = 98304;
 hipError_t launch_narrow(const double *src, float *dst, int64_t n, hipStream_t st);
 hipError_t launch_widen(const float *src, double *dst, int64_t n, hipStream_t st);
 
-// Fields of up to this many values are copied by a kernel between pinned memory
-// and the device, waited for by its count.  Upload and download, hipMemcpy /
-// so: 126 values 11.5 and 11.7 / 7.8 and 7.0 us, 1,000 14.5 and 14.7 / 8.2 and
-// 7.6, 2,198 8.9 and 8.5 / 9.0 and 8.5, 9,262 9.9 and 10.8 / 11.6 and 13.4 (it
-// takes another path above 16 KiB).
-constexpr int kSmallCopy = 2048;
-constexpr int kSmallWave = 128;                         // values per wave
-constexpr int kSmallWaves = kSmallCopy / kSmallWave;
-constexpr size_t kSmallCopyBytes = sizeof(double) * kSmallCopy + sizeof(uint32_t) * kSmallWaves;
+// Small fields are copied by a kernel between pinned memory and the device,
+// waited for by its counts, where hipMemcpy would take less than 16 KiB: it has
+// another path above that.  Upload and download, hipMemcpy / so, FP64: 512
+// values 12.4 and 12.6 / 8.5 and 8.1 us, 1,728 12.6 and 13.0 / 9.8 and 9.4, 4,096
+// 9.8 and 9.9 / 10.7 and 10.7; FP32 on the device: 4,096 12.9 and 13.4 / 11.7 and
+// 10.8, 8,000 10.4 and 10.8 / 12.8 and 12.6.  An ensemble with such a member
+// copies up to kMemberCopy values so, since hipMemcpy has to wait for the
+// stream, 8 us after a kernel: 11 fields of 24 members of 5..24, 3.50 and 3.70
+// ms / 2.82 and 2.72 (3.05 and 3.03 with its larger members by hipMemcpy).
+constexpr int kSmallWide = 2048, kSmallNarrow = 4096, kMemberCopy = 16384;
+constexpr int kSmallWave = 128; // values per wave
+constexpr size_t small_copy_bytes(int values) // pinned memory; values a multiple of kSmallWave
+{
+   return sizeof(double) * (size_t)values + sizeof(uint32_t) * (size_t)(values / kSmallWave);
+}
 
 // The copies of one context: not for two threads at a time, as the context.
 struct SmallCopy {
-   double *buffer = nullptr;   // kSmallCopyBytes of pinned memory, counts zero
+   int wide = kSmallWide, narrow = kSmallNarrow; // largest fields, FP64 and FP32 on the device
+   double *buffer = nullptr;
    uint32_t *counts = nullptr;
    uint32_t seq = 0;
-   void init(void *pinned);
-   // Complete on return; after the stream's earlier work.  narrow: the device's
-   // values are FP32.
-   hipError_t upload(const double *host, void *device, bool narrow, int n, hipStream_t st);
-   hipError_t download(const void *device, double *host, bool narrow, int n, hipStream_t st);
+   void init(void *pinned); // small_copy_bytes(narrow), aligned to 16
+   bool takes(size_t n, bool fp32) const { return n <= (size_t)(fp32 ? narrow : wide); }
+   // Complete on return; after the stream's earlier work.
+   hipError_t upload(const double *host, void *device, bool fp32, int n, hipStream_t st);
+   hipError_t download(void *device, double *host, bool fp32, int n, hipStream_t st);
 
  private:
    hipError_t wait(int n, hipStream_t st);

@@ -31,29 +31,35 @@ hipError_t launch(const S *src, D *dst, int64_t n, hipStream_t st)
 }
 
 // A small field between pinned memory and the device: bound by the latency of
-// the link, so one wave a workgroup and two values a lane, all loads at once
-// on many CUs (a workgroup of 1,024 threads instead: 1,000 values 14.4 up, 12.3
-// down).  Each wave stores its count when its values are where they belong.
-template <typename S, typename D>
-__global__ void __launch_bounds__(64) k_small(const S *__restrict__ src, D *__restrict__ dst, int n,
+// the link, so one wave a workgroup and two values a lane, 16 bytes of the
+// link, all of them in flight at once on many CUs (a workgroup of 1,024
+// threads instead: 1,000 values 14.4 us up, 12.3 down).  Each wave stores its
+// count when its values are where they belong.
+template <bool kUpload, typename T>
+__global__ void __launch_bounds__(64) k_small(double2 *__restrict__ pinned, T *__restrict__ device, int n,
                                               uint32_t *counts, uint32_t seq)
 {
-   const int i = (int)blockIdx.x * kSmallWave + (int)threadIdx.x, j = i + 64;
-   S a{}, b{};
-   if (i < n) a = src[i];
-   if (j < n) b = src[j];
-   if (i < n) dst[i] = (D)a;
-   if (j < n) dst[j] = (D)b;
+   const int pair = (int)blockIdx.x * 64 + (int)threadIdx.x, i = 2 * pair;
+   if (i < n) {
+      const bool two = i + 1 < n;
+      if constexpr (kUpload) {
+         const double2 v = pinned[pair]; // the buffer holds an even number of values
+         device[i] = (T)v.x;
+         if (two) device[i + 1] = (T)v.y;
+      } else {
+         pinned[pair] = double2{(double)device[i], two ? (double)device[i + 1] : 0.0};
+      }
+   }
    if (threadIdx.x == 0)
       __hip_atomic_store(counts + blockIdx.x, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-template <typename S, typename D>
-hipError_t launch_small(const S *src, D *dst, int n, uint32_t *counts, uint32_t seq, hipStream_t st)
+template <bool kUpload, typename T>
+hipError_t launch_small(double *pinned, T *device, int n, uint32_t *counts, uint32_t seq, hipStream_t st)
 {
    if (n <= 0) return hipSuccess;
-   hipLaunchKernelGGL((k_small<S, D>), dim3((unsigned)((n + kSmallWave - 1) / kSmallWave)), dim3(64), 0,
-                      st, src, dst, n, counts, seq);
+   hipLaunchKernelGGL((k_small<kUpload, T>), dim3((unsigned)((n + kSmallWave - 1) / kSmallWave)), dim3(64), 0,
+                      st, reinterpret_cast<double2 *>(pinned), device, n, counts, seq);
    return hipGetLastError();
 }
 
@@ -62,8 +68,8 @@ hipError_t launch_small(const S *src, D *dst, int n, uint32_t *counts, uint32_t 
 void SmallCopy::init(void *pinned)
 {
    buffer = static_cast<double *>(pinned);
-   counts = reinterpret_cast<uint32_t *>(buffer + kSmallCopy);
-   std::fill(counts, counts + kSmallWaves, 0u);
+   counts = reinterpret_cast<uint32_t *>(buffer + narrow);
+   std::fill(counts, counts + narrow / kSmallWave, 0u);
 }
 
 hipError_t SmallCopy::wait(int n, hipStream_t st)
@@ -73,20 +79,20 @@ hipError_t SmallCopy::wait(int n, hipStream_t st)
    return hipSuccess;
 }
 
-hipError_t SmallCopy::upload(const double *host, void *device, bool narrow, int n, hipStream_t st)
+hipError_t SmallCopy::upload(const double *host, void *device, bool fp32, int n, hipStream_t st)
 {
    std::memcpy(buffer, host, sizeof(double) * (size_t)n);
    ++seq;
-   const hipError_t e = narrow ? launch_small(buffer, static_cast<float *>(device), n, counts, seq, st)
-                               : launch_small(buffer, static_cast<double *>(device), n, counts, seq, st);
+   const hipError_t e = fp32 ? launch_small<true>(buffer, static_cast<float *>(device), n, counts, seq, st)
+                               : launch_small<true>(buffer, static_cast<double *>(device), n, counts, seq, st);
    return e == hipSuccess ? wait(n, st) : e;
 }
 
-hipError_t SmallCopy::download(const void *device, double *host, bool narrow, int n, hipStream_t st)
+hipError_t SmallCopy::download(void *device, double *host, bool fp32, int n, hipStream_t st)
 {
    ++seq;
-   const hipError_t e = narrow ? launch_small(static_cast<const float *>(device), buffer, n, counts, seq, st)
-                               : launch_small(static_cast<const double *>(device), buffer, n, counts, seq, st);
+   const hipError_t e = fp32 ? launch_small<false>(buffer, static_cast<float *>(device), n, counts, seq, st)
+                               : launch_small<false>(buffer, static_cast<double *>(device), n, counts, seq, st);
    if (e != hipSuccess) return e;
    const hipError_t w = wait(n, st);
    if (w == hipSuccess) std::memcpy(host, buffer, sizeof(double) * (size_t)n);

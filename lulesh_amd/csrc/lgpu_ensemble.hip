@@ -664,7 +664,9 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    if (!ok) return bail(LGPU_EDEVICE);
    if (e->brick) pick_brick_kernels(e);
    if (e->brick && build_brick_tables(e) != LGPU_OK) return bail(LGPU_EDEVICE);
-   if (hipHostMalloc((void **)&e->host, kSmallCopyBytes + (size_t)nMembers * (9 * 8 + 8) + 64 +
+   for (int32_t m = 0; m < nMembers; ++m)
+      if (e->elemCount[(size_t)m] <= kSmallWide) e->small.wide = e->small.narrow = kMemberCopy;
+   if (hipHostMalloc((void **)&e->host, small_copy_bytes(e->small.narrow) + (size_t)nMembers * (9 * 8 + 8) + 64 +
                                             (size_t)nMembers * kNumErrSites * 4,
                      hipHostMallocDefault) != hipSuccess)
       return bail(LGPU_ENOMEM);
@@ -694,7 +696,7 @@ int lgpu_ensemble_upload(lgpu_ensemble *e, int32_t member, int field, const doub
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
    void *dst = narrow ? (void *)(reinterpret_cast<float *>(base) + off) : (void *)(base + off);
-   if ((int64_t)n <= kSmallCopy) {
+   if (e->small.takes(n, narrow)) {
       ENS_HIP(e, e->small.upload(host, dst, narrow, (int)n, e->stream));
       return LGPU_OK;
    }
@@ -722,15 +724,15 @@ int lgpu_ensemble_download(lgpu_ensemble *e, int32_t member, int field, double *
    if (!base) return LGPU_EINVAL;
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
-   const void *src = narrow ? (const void *)(reinterpret_cast<float *>(base) + off) : (const void *)(base + off);
-   if ((int64_t)n <= kSmallCopy) {
+   void *src = narrow ? (void *)(reinterpret_cast<float *>(base) + off) : (void *)(base + off);
+   if (e->small.takes(n, narrow)) {
       ENS_HIP(e, e->small.download(src, host, narrow, (int)n, e->stream));
       return LGPU_OK;
    }
    ENS_HIP(e, hipStreamSynchronize(e->stream));
    if (narrow && (int64_t)n > kConvertOnHost) {
       double *wide = scratch_doubles(e);
-      ENS_HIP(e, launch_widen(static_cast<const float *>(src), wide, (int64_t)n, e->stream));
+      ENS_HIP(e, launch_widen(static_cast<float *>(src), wide, (int64_t)n, e->stream));
       ENS_HIP(e, hipStreamSynchronize(e->stream));
       ENS_HIP(e, hipMemcpy(host, wide, 8 * n, hipMemcpyDeviceToHost));
    } else if (narrow) {
@@ -748,7 +750,7 @@ int lgpu_ensemble_run(lgpu_ensemble *e, lgpu_time_state *ts, int32_t maxCycle, i
    if (!e || !ts) return LGPU_EINVAL;
    const int M = e->nMembers;
    // Pinned staging: 9 double arrays, cycle, active, err.
-   double *hd = reinterpret_cast<double *>(e->host + kSmallCopyBytes);
+   double *hd = reinterpret_cast<double *>(e->host + small_copy_bytes(e->small.narrow));
    int32_t *hcyc = reinterpret_cast<int32_t *>(hd + 9 * (size_t)M);
    int32_t *hact = hcyc + M;
    int32_t *herr = hact + M;

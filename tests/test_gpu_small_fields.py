@@ -1,5 +1,5 @@
-"""Fields of up to 2,048 values travel by a kernel through pinned memory: the
-same bits as the copies of larger fields, after the stream's earlier work.
+"""Small fields travel by a kernel through pinned memory: the same bits as the
+copies of larger fields, after the stream's earlier work.
 """
 import ctypes
 
@@ -16,7 +16,7 @@ def _bits(n, seed):
     return v.view(np.float64)
 
 
-# one value, whole and part waves of 128, nodes or elements beyond 2,048
+# one value, whole and part waves of 128, beyond 2,048, of which single problems copy FP64 otherwise
 @pytest.mark.parametrize("s", [1, 4, 7, 11, 12, 13])
 def test_every_bit_comes_back(s):
     ctx = la.SedovDevice(s)
