@@ -412,9 +412,8 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    const int64_t nCorner = sp.nCorner;
    int cus = 0;
    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 0;
-   c->s.eosSplit = eos_split(sp.numElem) ? 1 : 0;
    // every group may end in a partly filled workgroup
-   const size_t eosBlocks = E / (size_t)(kEosBlock / (c->s.eosSplit ? kEosShare : 1)) + 4;
+   const size_t eosBlocks = E / (size_t)(kEosBlock / kEosShare) + 4;
 
    // Arena layout.
    struct Slot { void **dst; size_t bytes; };
@@ -533,10 +532,15 @@ int set_groups(lgpu_ctx *c, const std::vector<int32_t> &reps, const std::vector<
                const std::vector<int64_t> &sizes)
 {
    c->eosSlots.clear();
+   double repeats = 0.;
+   for (size_t g = 0; g < reps.size(); ++g) repeats += (double)reps[g] * (double)sizes[g];
    int64_t at = 0;
    for (size_t g = 0; g < reps.size(); ++g) {
       std::vector<EosSlot> slots;
-      add_eos_slots(slots, EosGroup{at, sizes[g], reps[g]}, c->s.eosSplit != 0);
+      const EosGroup group{at, sizes[g], reps[g]};
+      const bool shared = eos_shares(c->numElem, c->numElem, group, repeats, c->precision == LGPU_MIXED);
+      if (shared) c->s.eosSplit = 1;
+      add_eos_slots(slots, group, shared);
       size_t r = 0;
       for (const EosSlot &sl : slots) {
          const int64_t p = sl.pos - at;

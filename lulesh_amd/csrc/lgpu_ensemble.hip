@@ -503,11 +503,8 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    }
    // Offsets.
    DevState &s = e->s;
-   {
-      int64_t totE = 0;
-      for (int32_t m = 0; m < nMembers; ++m) totE += members[m].numElem;
-      s.eosSplit = eos_split(totE) ? 1 : 0;
-   }
+   int64_t totE = 0;
+   for (int32_t m = 0; m < nMembers; ++m) totE += members[m].numElem;
    e->nodeStart.assign((size_t)nMembers + 1, 0);
    e->elemStart.assign((size_t)nMembers + 1, 0);
    std::vector<int64_t> cornerStart((size_t)nMembers + 1, 0);
@@ -531,11 +528,16 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
          for (int32_t i = 0; i < d.regElemSize[r]; ++i) repOf[(size_t)d.regElemlist[r][i]] = rep;
       }
       std::sort(reps.begin(), reps.end(), std::greater<int32_t>());
+      double repeats = 0.;
+      for (int32_t rep : repOf) repeats += rep;
       for (int32_t rep : reps) {
          const int64_t pos = (int64_t)perm.size();
          for (int32_t el = 0; el < d.numElem; ++el)
             if (repOf[(size_t)el] == rep) perm.push_back(el + e0);
-         add_eos_slots(eosSlots, EosGroup{pos, (int64_t)perm.size() - pos, rep}, s.eosSplit != 0);
+         const EosGroup group{pos, (int64_t)perm.size() - pos, rep};
+         const bool shared = eos_shares(totE, d.numElem, group, repeats, prec == LGPU_MIXED);
+         if (shared) s.eosSplit = 1;
+         add_eos_slots(eosSlots, group, shared);
       }
       blockMember.resize(eosSlots.size(), m);
       blockStart.push_back((int32_t)eosSlots.size());

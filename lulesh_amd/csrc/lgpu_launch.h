@@ -26,23 +26,34 @@ struct EosGroup {
    int32_t rep;
 };
 
-// Threads that share an element's repeats, and the repeat count from which
-// they do, in launches that split (eos_split).
+// Threads that share an element's repeats in slots that share them.
 constexpr int kEosShare = 4;
-constexpr int kEosSplitReps = 8;
 
-// Whether k_eos shares the repeats of the heaviest elements between threads:
-// up to 2^20 elements, where a wave's 20 to 50 repeats in a row are a good part
-// of the launch.  One thread / shared: s=8 13.7 / 7.4 us, s=30 14.8 / 8.1, s=45
-// 15.6 / 11.6, s=63 mixed (50 repeats) 25.6 / 20.3, s=64 22.1 / 21.2, s=96 FMA
-// 44.7 / 43.0, s=101 50.6 / 49.9; above: 64 members, 6.0 M elements, 268 / 291,
-// s=192 299 / 341 (each sharing thread loads the operands again).
-inline bool eos_split(int64_t numElem) { return numElem <= (1 << 20); }
+// Whether the threads of a group's slots share its elements' repeats: a wave's
+// 10 to 50 repeats in a row are a good part of a short launch, but each sharing
+// thread loads the operands again.  So only counts well above the mean of the
+// problem (`repeats` in all), and the larger the launch, within which such
+// waves run beside the others, the more repeats the group has to hold: one per
+// element of the problem for 365,000 elements of the launch (mixed 150,000).
+// One thread / shared, us, 11 regions, FP64 and FP64_FMA: s=8 10 repeats 11.5 /
+// 9.5; s=30 10 12.9 / 10.0, 20 16.4 / 10.8; s=64 10 18.1 / 18.4, 50 34.1 / 32.0; s=81
+// 10 25.7 / 26.8; s=96 10 33.5 / 37.4, 20 43.9 / 44.2, 50 77.8 / 64.0; s=101 10 38.9 /
+// 42.4, 20 51.8 / 50.0, 50 93.8 / 73.1; s=128 20 84.7 / 99.9, 50 151 / 132; 5 regions:
+// s=101 10 51.8 / 50.5, 20 72.7 / 62.7, s=128 20 116 / 123; 21 regions: s=192 30 286 /
+// 333.  Mixed, 16 regions: s=63 10 15.5 / 14.8, 50 28.2 / 21.9; 21 regions: s=101 20
+// 30.2 / 35.1, 50 41.0 / 43.4.  Near the mean (9 for half of the elements): mixed
+// s=63 30.0 / 38.4, s=101 110 / 132.
+inline bool eos_shares(int64_t launchElems, int64_t numElem, const EosGroup &g, double repeats,
+                       bool mixed)
+{
+   return g.rep >= 8 && (double)g.rep * (double)numElem >= 2.0 * repeats &&
+          (double)g.rep * (double)g.count * (mixed ? 150e3 : 365e3) >= (double)launchElems * (double)numElem;
+}
 
 // The workgroups of one group.
-inline void add_eos_slots(std::vector<EosSlot> &slots, const EosGroup &g, bool split)
+inline void add_eos_slots(std::vector<EosSlot> &slots, const EosGroup &g, bool shared)
 {
-   const int share = split && g.rep >= kEosSplitReps ? kEosShare : 1, per = kEosBlock / share;
+   const int share = shared ? kEosShare : 1, per = kEosBlock / share;
    for (int64_t at = 0; at < g.count; at += per)
       slots.push_back(EosSlot{(int32_t)(g.pos + at), (int32_t)std::min<int64_t>(per, g.count - at),
                               g.rep, share});

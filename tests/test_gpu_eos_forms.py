@@ -49,8 +49,8 @@ def test_waves_between_the_volume_limits(precision, eosvmin, eosvmax):
 
 @pytest.mark.parametrize("s,regions,cost", [(1, 1, 0), (2, 11, 1), (5, 21, 4), (17, 11, 0), (50, 21, 2), (102, 21, 2)])
 def test_elements_phase_with_shared_and_single_threads(s, regions, cost):
-    """Up to 2^20 elements (all sizes here but 102) four threads share the
-    repeats of the heaviest elements, above that one thread runs them all: the
+    """Four threads share the repeats of the heaviest elements (here all sizes
+    but 1, 2 and 102), or one thread runs them all: the
     FP64 elements phase is the oracle's bit for bit on both sides of the line,
     on partly filled workgroups and with repeat counts below and above the
     count that is shared."""
