@@ -236,11 +236,11 @@ enum lgpu_option {
                                      16 (16x16 element columns, default) or 8
                                      (16x8)                                  */
    LGPU_OPT_EOS_INTERLEAVE = 9    /* k_eos dispatch order: 0 work-list order,
-                                     largest EOS repeat count first; k > 0
-                                     (default 4) one workgroup of the largest
-                                     count every k+1 dispatches (an odd k is
-                                     raised by one: the 8 XCDs are dealt
-                                     workgroups in turn)                    */
+                                     largest EOS repeat count first; k > 0 one
+                                     workgroup of the largest count every k+1
+                                     dispatches (an odd k is raised by one: the
+                                     8 XCDs are dealt workgroups in turn).
+                                     Default: 0, 2 or 4, by size and regions */
 };
 int lgpu_set_option(lgpu_ctx *ctx, int option, int64_t value);
 /* Current value of an option (the brick chunks report the defaults chosen at

@@ -63,7 +63,8 @@ struct lgpu_ctx {
    std::vector<PlacedSlot> eosSlots; // in work-list order
    int eosInterleave = 0;
    int32_t brickPerCu = 0;
-   int64_t brickSlots = 0, genericSlots = 0; // resident workgroups: nodal brick kernels, k_force
+   // resident workgroups: nodal brick kernels, k_force, k_eos
+   int64_t brickSlots = 0, genericSlots = 0, eosResident = 0;
    bool timing = false;
    uint32_t timingMask = 0xffffffffu;
    Consts k{};
@@ -251,6 +252,24 @@ int set_eos_order(lgpu_ctx *c, int k)
                               sizeof(EosSlot) * slots.size(), hipMemcpyHostToDevice));
    c->eosInterleave = std::max(0, k);
    return LGPU_OK;
+}
+
+// The default order: work-list order where all workgroups are resident at once,
+// the longest started first; otherwise one workgroup of the largest repeat
+// count every 5 dispatches, or every 3 where these are more than a fifth of
+// all, so that they have started well before the end.  Every 5 / every 3 /
+// work-list order, us: s=45 14.5 / 14.0 / 13.3; s=63 mixed (16 regions, 50
+// repeats) 22.0 / 22.1 / 19.5; s=101 of 5 regions 51.1 / 50.2 / 51.4, of 11, shared
+// between threads, 50.6 / 47.7 / 49.8; s=192 of 5 281 / 253 / 295 (20 repeats 322 /
+// 299 / 390), of 11 262 / 272 / 340, of 21 287 / 296 / 346; mixed of 5 220 / 204 / 246,
+// of 11 190 / 194 / 228.
+int default_interleave(const lgpu_ctx *c)
+{
+   const int64_t all = (int64_t)c->eosSlots.size();
+   if (all == 0 || all <= c->eosResident) return 0;
+   int64_t heavy = 0;
+   while (heavy < all && c->eosSlots[(size_t)heavy].slot.rep == c->eosSlots[0].slot.rep) ++heavy;
+   return 5 * heavy > all ? 2 : 4;
 }
 
 // Device array of a field.  `narrow`: stored as FP32 in the mixed form (the
@@ -480,6 +499,7 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
    s.xcdRemap = 1;
    s.isBrick = brick ? 1 : 0;
    c->genericSlots = (int64_t)cus * 2;
+   c->eosResident = (int64_t)cus * (sp.precision == LGPU_MIXED ? PolicyMixed::kEosWaves : PolicyFp64::kEosWaves);
    s.brickFaces = (brick && sp.brickFaces) ? 1 : 0;
    if (brick) {
       Brick &g = s.brick;
@@ -556,10 +576,7 @@ int set_groups(lgpu_ctx *c, const std::vector<int32_t> &reps, const std::vector<
 // read-back buffers.
 int finish_context(lgpu_ctx *c)
 {
-   // One workgroup of the largest repeat count every 5 dispatches: measured
-   // 7-10% faster than plain work-list order at s=192 (FP64, 11 and 21
-   // regions).
-   const int st = set_eos_order(c, 4);
+   const int st = set_eos_order(c, default_interleave(c));
    if (st != LGPU_OK) return st;
    constexpr size_t kSmallAt = (64 + sizeof(DevTime) + 63) / 64 * 64;
    if (hipHostMalloc((void **)&c->hostDt, kSmallAt + small_copy_bytes(kSmallNarrow), hipHostMallocDefault) !=
