@@ -239,6 +239,37 @@ inline void pick_member_tile(Brick &g)
    set_brick_tile(g, bestW, 256 / bestW);
 }
 
+// One problem's walk takes other tiles than 16 x 16 threads.
+inline bool other_tile(const Brick &g) { return g.tileW != 16 || (g.rows != 16 && g.rows != 8); }
+
+// walk_cost of the tile and chunk chosen; a plane takes 7% longer where the
+// tile's width is read at run time (one problem's s=64 FP64: 34.9 us for 20
+// columns in chunks of 3, k_nodal_block 33.5).
+inline double brick_walk_cost(const Brick &g, int slots)
+{
+   if (slots < 1) return 0.;
+   const double cost = walk_cost((int64_t)g.tilesX * g.tilesY, g.en, slots, g.chunkZ);
+   return other_tile(g) ? 1.07 * cost : cost;
+}
+
+// The fused nodal kernel's tile and chunk for one problem: 16 x 16 threads, or
+// the tile that an ensemble's member of this size would have where that needs
+// 7% fewer columns and the walk is 7% shorter by more than its planes cost.
+// 16 x 16 / that, us, FP64: s=75 54.8 / 49.0, s=90 75.5 / 65.0, s=95 80.3 / 70.2,
+// s=105 112.9 / 100.7, s=120 162 / 152, s=125 171 / 155; FP64_FMA s=90 60.6 / 54.1,
+// s=120 132 / 129; mixed s=75 34.5 / 29.2, s=105 63.5 / 62.5, s=125 126 / 121; not
+// taken: s=84 (35 columns of 36) 54.7 / 56.1, s=110 111.7 / 111.9, FP64_FMA s=140
+// 187 / 196.
+inline void pick_brick_walk(Brick &g, int slots)
+{
+   set_brick_chunk(g, pick_brick_chunk(g, slots, 1));
+   Brick other = g;
+   pick_member_tile(other);
+   set_brick_chunk(other, pick_brick_chunk(other, slots, 1));
+   const double columns = (double)g.tilesX * g.tilesY, fewer = (double)other.tilesX * other.tilesY;
+   if (fewer <= 0.93 * columns && brick_walk_cost(other, slots) < brick_walk_cost(g, slots)) g = other;
+}
+
 // Kinematics tiles of w x h elements (one per thread of a 256-thread
 // workgroup), kept within the LDS of the 16 x 16 tile: (h+1) node rows of
 // 2 ceil((w+1)/2) values, at most 17 x 18.
