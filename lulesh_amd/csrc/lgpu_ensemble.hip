@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <functional>
@@ -316,6 +317,37 @@ int32_t equal_blocks(const std::vector<int64_t> &counts, std::vector<MemberBlock
    return (int32_t)blocks.size();
 }
 
+// k_eos's dispatch order over all members: heavy workgroups (kEosHeavyReps
+// repeats on) first where all are resident at once, and otherwise one of them
+// every 3 dispatches, so that they have started well before the end; both kinds
+// by member.  By member throughout, each one's heavy ones first / every 3 / every
+// 5 / heavy first, us: 64 members of 16..64, FP64, 267 / 262 / 274 / 293; 16 of
+// 40..90, FP64_FMA, 284 / 281 / 272 / 312; mixed 40 of 20..50 87 / 78 / 88 / 84; 24
+// of 5..24 (resident) 17.0 / 18.2 / 17.3 / 16.2.
+constexpr int kEosHeavyReps = 8;
+
+void order_eos_blocks(std::vector<EosSlot> &slots, std::vector<EosBlock> &blocks, int64_t resident)
+{
+   std::vector<size_t> heavy, rest, order;
+   for (size_t b = 0; b < slots.size(); ++b)
+      (slots[b].rep >= kEosHeavyReps ? heavy : rest).push_back(b);
+   const size_t between = (int64_t)slots.size() <= resident ? 0 : 2;
+   size_t r = 0;
+   for (size_t b : heavy) {
+      order.push_back(b);
+      for (size_t j = 0; j < between && r < rest.size(); ++j) order.push_back(rest[r++]);
+   }
+   order.insert(order.end(), rest.begin() + (std::ptrdiff_t)r, rest.end());
+   std::vector<EosSlot> s2;
+   std::vector<EosBlock> b2;
+   for (size_t b : order) {
+      s2.push_back(slots[b]);
+      b2.push_back(blocks[b]);
+   }
+   slots.swap(s2);
+   blocks.swap(b2);
+}
+
 // Member tables of the brick path for the current kernel and chunk choices:
 // per-member bricks with offsets, and the kernels' workgroups.
 int build_brick_tables(lgpu_ensemble *e)
@@ -510,7 +542,8 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    std::vector<int64_t> cornerStart((size_t)nMembers + 1, 0);
    // The EOS work list, as for a single domain: each member's elements grouped
    // by EOS repeat count, largest first, in mesh order within a group.
-   std::vector<int32_t> perm, blockMember, blockStart(1, 0);
+   std::vector<int32_t> perm, blockStart(1, 0);
+   std::vector<EosBlock> eosBlock;
    std::vector<EosSlot> eosSlots;
    for (int32_t m = 0; m < nMembers; ++m) {
       const lgpu_mesh_desc &d = members[m];
@@ -539,8 +572,17 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
          if (shared) s.eosSplit = 1;
          add_eos_slots(eosSlots, group, shared);
       }
-      blockMember.resize(eosSlots.size(), m);
+      for (size_t b = eosBlock.size(); b < eosSlots.size(); ++b)
+         eosBlock.push_back(EosBlock{m, (int32_t)b});
       blockStart.push_back((int32_t)eosSlots.size());
+   }
+   {
+      int dev = 0, cus = 0;
+      if (hipGetDevice(&dev) != hipSuccess ||
+          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+         cus = 0;
+      order_eos_blocks(eosSlots, eosBlock,
+                       (int64_t)cus * (prec == LGPU_MIXED ? PolicyMixed::kEosWaves : PolicyFp64::kEosWaves));
    }
    const size_t E = (size_t)e->elemStart[nMembers], N = (size_t)e->nodeStart[nMembers];
    const size_t nCorner = (size_t)cornerStart[nMembers];
@@ -593,7 +635,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    add((void **)&s.dtOut, 16);
    add((void **)&s.memberNodeStart, 4 * ((size_t)nMembers + 1));
    add((void **)&s.memberElemStart, 4 * ((size_t)nMembers + 1));
-   add((void **)&s.blockMember, 4 * (size_t)blockStart[nMembers]);
+   add((void **)&s.eosBlock, sizeof(EosBlock) * (size_t)blockStart[nMembers]);
    add((void **)&s.eosSlot, sizeof(EosSlot) * (size_t)blockStart[nMembers]);
    add((void **)&s.memberBlockStart, 4 * ((size_t)nMembers + 1));
    size_t total = 0, stateBytes = 0;
@@ -659,7 +701,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
              h2d((void *)s.nodeBC, bc.data(), N) &&
              h2d((void *)s.memberNodeStart, e->nodeStart.data(), 4 * e->nodeStart.size()) &&
              h2d((void *)s.memberElemStart, e->elemStart.data(), 4 * e->elemStart.size()) &&
-             h2d((void *)s.blockMember, blockMember.data(), 4 * blockMember.size()) &&
+             h2d((void *)s.eosBlock, eosBlock.data(), sizeof(EosBlock) * eosBlock.size()) &&
              h2d((void *)s.eosSlot, eosSlots.data(), sizeof(EosSlot) * eosSlots.size()) &&
              h2d((void *)s.memberBlockStart, blockStart.data(), 4 * blockStart.size()) &&
              h2d(s.v, ones.data(), 8 * E);

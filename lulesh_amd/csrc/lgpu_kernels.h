@@ -199,6 +199,12 @@ struct MemberBrick {
    int32_t nodeOff, elemOff;
 };
 
+// A k_eos workgroup's member in an ensemble, and its dt partial, which are by
+// member whatever the order of the workgroups.
+struct EosBlock {
+   int32_t member, partial;
+};
+
 // One workgroup of a brick kernel in an ensemble.
 struct MemberBlock {
    int32_t member;
@@ -283,7 +289,7 @@ struct DevState {
    const double *memberDt;         // per-member deltatime
    const int32_t *memberActive;    // per-member loop flag
    int32_t *memberErr;             // nMembers x kNumErrSites
-   const int32_t *blockMember;     // k_eos block -> member
+   const EosBlock *eosBlock;       // k_eos block -> member and dt partial
    const int32_t *memberBlockStart; // nMembers+1: k_eos blocks of each member
    double *memberDtOut;            // 2 per member: dtcourant, dthydro
    EnsTime ensTime;                // the members' next TimeIncrement
