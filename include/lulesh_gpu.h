@@ -225,16 +225,21 @@ enum lgpu_option {
                                      kernels of the generic path: 64, 128
                                      or 256                                  */
    LGPU_OPT_BRICK_CHUNK = 4,      /* node planes per workgroup of the fused
-                                     brick kernel (1..mesh edge)             */
+                                     brick kernel (1..mesh edge); setting it
+                                     selects the kernel that walks up columns,
+                                     also where a small brick has another     */
    LGPU_OPT_XCD_REMAP = 5,        /* 1 (default): contiguous block ranges per
                                      XCD; 0: hardware order                 */
    LGPU_OPT_KERNEL_TIMING_MASK = 6, /* bit k: time kernel k while timing is on
                                      (default: all)                          */
    LGPU_OPT_KIN_CHUNK = 7,        /* element planes per workgroup of the
-                                     brick kinematics kernel (1..mesh edge)  */
+                                     brick kinematics kernel (1..mesh edge);
+                                     setting it selects the column walk       */
    LGPU_OPT_BRICK_ROWS = 8,       /* thread rows of a fused brick workgroup:
-                                     16 (16x16 element columns, default) or 8
-                                     (16x8)                                  */
+                                     16 (16x16 element columns, or by default
+                                     another shape of 256 threads where it
+                                     covers the mesh with fewer) or 8 (16x8);
+                                     setting it selects the column walk       */
    LGPU_OPT_EOS_INTERLEAVE = 9    /* k_eos dispatch order: 0 work-list order,
                                      largest EOS repeat count first; k > 0 one
                                      workgroup of the largest count every k+1
@@ -308,17 +313,20 @@ enum lgpu_ensemble_option {
    LGPU_ENS_OPT_BLOCK_KIN = 5,
    LGPU_ENS_OPT_XCD_REMAP = 6,
    LGPU_ENS_OPT_BRICK_CHUNK = 7,  /* brick path: node planes per workgroup of
-                                     the fused nodal kernel, every member      */
+                                     the fused nodal kernel, every member;
+                                     selects the kernel that walks up columns */
    LGPU_ENS_OPT_KIN_CHUNK = 8,    /* brick path: element planes per
-                                     workgroup of the kinematics kernel       */
+                                     workgroup of the kinematics kernel;
+                                     selects the column walk                  */
    LGPU_ENS_OPT_PATH = 9          /* read only: 1 brick path, 0 CSR gathers   */
 };
 int lgpu_ensemble_set_option(lgpu_ensemble *ens, int option, int64_t value);
 int lgpu_ensemble_get_option(lgpu_ensemble *ens, int option, int64_t *value);
 
 /* Autotuner: times trial cycles of this ensemble for each candidate block
- * shape of the force, node and kinematics kernels and for both XCD block
- * mappings, keeps the fastest, and restores the state afterwards. */
+ * shape of the force, node and kinematics kernels (brick path: the small-brick
+ * kernels and the chunks of the column walks) and for both XCD block mappings,
+ * keeps the fastest, and restores the state afterwards. */
 int lgpu_ensemble_autotune(lgpu_ensemble *ens, const lgpu_time_state *ts, int32_t trial_cycles);
 
 int lgpu_ensemble_num_kernels(void);

@@ -579,7 +579,9 @@ int finish_context(lgpu_ctx *c)
    const int st = set_eos_order(c, default_interleave(c));
    if (st != LGPU_OK) return st;
    constexpr size_t kSmallAt = (64 + sizeof(DevTime) + 63) / 64 * 64;
-   if (hipHostMalloc((void **)&c->hostDt, kSmallAt + small_copy_bytes(kSmallNarrow), hipHostMallocDefault) !=
+   if (copies_by_kernel({c->numNode}, {c->numElem}, kSmallProblem, c->precision == LGPU_MIXED))
+      c->small.limit = kSmallProblem;
+   if (hipHostMalloc((void **)&c->hostDt, kSmallAt + small_copy_bytes(c->small.limit), hipHostMallocDefault) !=
        hipSuccess)
       return LGPU_ENOMEM;
    c->hostErr = reinterpret_cast<int32_t *>(c->hostDt + 2);
@@ -885,7 +887,7 @@ int lgpu_upload(lgpu_ctx *c, int field, const double *host)
    double *dst = real_field_ptr(c, field, isElem, narrow);
    if (!dst) return LGPU_EINVAL;
    const size_t n = isElem ? (size_t)c->numElem : (size_t)c->numNode;
-   if (c->small.takes(n, narrow)) {
+   if (c->small.takes(n)) {
       HIP_OR_RETURN(c, c->small.upload(host, dst, narrow, (int)n, c->stream));
       return LGPU_OK;
    }
@@ -911,7 +913,7 @@ int lgpu_download(lgpu_ctx *c, int field, double *host)
    bool isElem, narrow;
    double *src = real_field_ptr(c, field, isElem, narrow);
    const size_t n = isElem ? (size_t)c->numElem : (size_t)c->numNode;
-   if (src && c->small.takes(n, narrow)) {
+   if (src && c->small.takes(n)) {
       HIP_OR_RETURN(c, c->small.download(src, host, narrow, (int)n, c->stream));
       return LGPU_OK;
    }

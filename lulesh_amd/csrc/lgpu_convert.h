@@ -6,6 +6,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+#include <vector>
+
 namespace lgpu {
 
 // Fields of up to this many values are converted on the host, where a launch
@@ -18,30 +21,51 @@ hipError_t launch_narrow(const double *src, float *dst, int64_t n, hipStream_t s
 hipError_t launch_widen(const float *src, double *dst, int64_t n, hipStream_t st);
 
 // Small fields are copied by a kernel between pinned memory and the device,
-// waited for by its counts, where hipMemcpy would take less than 16 KiB: it has
-// another path above that.  Upload and download, hipMemcpy / so, FP64: 512
-// values 12.4 and 12.6 / 8.5 and 8.1 us, 1,728 12.6 and 13.0 / 9.8 and 9.4, 4,096
-// 9.8 and 9.9 / 10.7 and 10.7; FP32 on the device: 4,096 12.9 and 13.4 / 11.7 and
-// 10.8, 8,000 10.4 and 10.8 / 12.8 and 12.6.  An ensemble with such a member
-// copies up to kMemberCopy values so, since hipMemcpy has to wait for the
-// stream, 8 us after a kernel: 11 fields of 24 members of 5..24, 3.50 and 3.70
-// ms / 2.82 and 2.72 (3.05 and 3.03 with its larger members by hipMemcpy).
-constexpr int kSmallWide = 2048, kSmallNarrow = 4096, kMemberCopy = 16384;
+// waited for by its counts: hipMemcpy takes 12 us below 16 KiB and another path
+// above.  Upload and download, hipMemcpy / so: 512 values 12.4 and 12.6 / 8.5 and
+// 8.1 us, 1,728 12.6 and 13.0 / 9.8 and 9.4, 4,096 9.8 and 9.9 / 10.7 and 10.7, 8,000
+// 10.3 and 11.3 / 12.1 and 12.7, 13,824 11.3 and 13.2 / 14.8 and 16.5.  hipMemcpy has
+// to wait for the stream, 9 us after a kernel, so a context copies all of its
+// fields one way (copies_by_kernel): 24 members of 5..24, 11 fields, hipMemcpy
+// 3.50 and 3.70 ms, members of up to 2,048 elements so 3.05 and 3.03, all 2.82 and
+// 2.72.
+constexpr int kSmallProblem = 4096, kSmallMembers = 16384; // largest fields
 constexpr int kSmallWave = 128; // values per wave
 constexpr size_t small_copy_bytes(int values) // pinned memory; values a multiple of kSmallWave
 {
    return sizeof(double) * (size_t)values + sizeof(uint32_t) * (size_t)(values / kSmallWave);
 }
 
+// Whether the kernel takes less time over the 6 node and 5 element fields of a
+// state, for each problem's nodes and elements; those above `limit` go by
+// hipMemcpy in any case.  fp32: 3 of the element fields are FP32 on the device.
+inline bool copies_by_kernel(const std::vector<int32_t> &nodes, const std::vector<int32_t> &elems, int limit,
+                             bool fp32)
+{
+   double kernel = 0., memcpy = 0.; // us
+   auto add = [&](double fields, double n, double bytes) {
+      const double m = n * bytes <= 16384. ? 12.4 : 8.7 + 0.00025 * n;
+      const double k = 7.6 + 0.0008 * std::min(n, 4096.) + 0.0005 * std::max(n - 4096., 0.);
+      memcpy += fields * m;
+      kernel += fields * (n <= limit ? k : m + 9.0);
+   };
+   for (int32_t n : nodes) add(6., n, 8.);
+   for (int32_t n : elems) {
+      add(2., n, 8.);
+      add(3., n, fp32 ? 4. : 8.);
+   }
+   return kernel < memcpy;
+}
+
 // The copies of one context: not for two threads at a time, as the context.
 struct SmallCopy {
-   int wide = kSmallWide, narrow = kSmallNarrow; // largest fields, FP64 and FP32 on the device
+   int limit = 0; // largest field, 0 where hipMemcpy copies all
    double *buffer = nullptr;
    uint32_t *counts = nullptr;
    uint32_t seq = 0;
-   void init(void *pinned); // small_copy_bytes(narrow), aligned to 16
-   bool takes(size_t n, bool fp32) const { return n <= (size_t)(fp32 ? narrow : wide); }
-   // Complete on return; after the stream's earlier work.
+   void init(void *pinned); // small_copy_bytes(limit), aligned to 16
+   bool takes(size_t n) const { return n <= (size_t)limit; }
+   // Complete on return; after the stream's earlier work.  fp32: on the device.
    hipError_t upload(const double *host, void *device, bool fp32, int n, hipStream_t st);
    hipError_t download(void *device, double *host, bool fp32, int n, hipStream_t st);
 

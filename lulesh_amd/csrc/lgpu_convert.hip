@@ -68,8 +68,8 @@ hipError_t launch_small(double *pinned, T *device, int n, uint32_t *counts, uint
 void SmallCopy::init(void *pinned)
 {
    buffer = static_cast<double *>(pinned);
-   counts = reinterpret_cast<uint32_t *>(buffer + narrow);
-   std::fill(counts, counts + narrow / kSmallWave, 0u);
+   counts = reinterpret_cast<uint32_t *>(buffer + limit);
+   std::fill(counts, counts + limit / kSmallWave, 0u);
 }
 
 hipError_t SmallCopy::wait(int n, hipStream_t st)

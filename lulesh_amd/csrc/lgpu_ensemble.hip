@@ -708,9 +708,9 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    if (!ok) return bail(LGPU_EDEVICE);
    if (e->brick) pick_brick_kernels(e);
    if (e->brick && build_brick_tables(e) != LGPU_OK) return bail(LGPU_EDEVICE);
-   for (int32_t m = 0; m < nMembers; ++m)
-      if (e->elemCount[(size_t)m] <= kSmallWide) e->small.wide = e->small.narrow = kMemberCopy;
-   if (hipHostMalloc((void **)&e->host, small_copy_bytes(e->small.narrow) + (size_t)nMembers * (9 * 8 + 8) + 64 +
+   if (copies_by_kernel(e->nodeCount, e->elemCount, kSmallMembers, prec == LGPU_MIXED))
+      e->small.limit = kSmallMembers;
+   if (hipHostMalloc((void **)&e->host, small_copy_bytes(e->small.limit) + (size_t)nMembers * (9 * 8 + 8) + 64 +
                                             (size_t)nMembers * kNumErrSites * 4,
                      hipHostMallocDefault) != hipSuccess)
       return bail(LGPU_ENOMEM);
@@ -740,7 +740,7 @@ int lgpu_ensemble_upload(lgpu_ensemble *e, int32_t member, int field, const doub
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
    void *dst = narrow ? (void *)(reinterpret_cast<float *>(base) + off) : (void *)(base + off);
-   if (e->small.takes(n, narrow)) {
+   if (e->small.takes(n)) {
       ENS_HIP(e, e->small.upload(host, dst, narrow, (int)n, e->stream));
       return LGPU_OK;
    }
@@ -769,7 +769,7 @@ int lgpu_ensemble_download(lgpu_ensemble *e, int32_t member, int field, double *
    const size_t n = isElem ? (size_t)e->elemCount[member] : (size_t)e->nodeCount[member];
    const size_t off = isElem ? (size_t)e->elemStart[member] : (size_t)e->nodeStart[member];
    void *src = narrow ? (void *)(reinterpret_cast<float *>(base) + off) : (void *)(base + off);
-   if (e->small.takes(n, narrow)) {
+   if (e->small.takes(n)) {
       ENS_HIP(e, e->small.download(src, host, narrow, (int)n, e->stream));
       return LGPU_OK;
    }
@@ -794,7 +794,7 @@ int lgpu_ensemble_run(lgpu_ensemble *e, lgpu_time_state *ts, int32_t maxCycle, i
    if (!e || !ts) return LGPU_EINVAL;
    const int M = e->nMembers;
    // Pinned staging: 9 double arrays, cycle, active, err.
-   double *hd = reinterpret_cast<double *>(e->host + small_copy_bytes(e->small.narrow));
+   double *hd = reinterpret_cast<double *>(e->host + small_copy_bytes(e->small.limit));
    int32_t *hcyc = reinterpret_cast<int32_t *>(hd + 9 * (size_t)M);
    int32_t *hact = hcyc + M;
    int32_t *herr = hact + M;

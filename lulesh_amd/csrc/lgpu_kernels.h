@@ -1,6 +1,6 @@
 // lgpu_kernels.h -- device kernels of the Lagrange leapfrog step.
 //
-// Four passes per cycle, each a single launch over its whole index space:
+// The passes of a cycle, each a single launch over its whole index space:
 //
 //   k_force  (elements)  stress integration + Flanagan-Belytschko hourglass,
 //                        per-corner forces to corner planes
@@ -11,9 +11,15 @@
 //   k_eos    (region-ordered elements)  qstop check, monotonic-Q limiter,
 //                        delv = vnew - v, EOS with its region repeat count,
 //                        sound speed, volume update, Courant/hydro block minima
-//   k_dt_slots / k_dt_reduce (one block per problem) Courant/hydro minima
-//                        over the k_eos slots (one problem: atomic minima
-//                        into 256 slot pairs) or block partials (ensembles)
+//                        (one problem: by atomic minima into 256 slot pairs)
+//   k_dt_slots           host-driven cycles: Courant/hydro minima of the slots
+//   k_begin_cycle        device loop: the same, and TimeIncrement, as the next
+//                        cycle begins; in short cycles in its first kernel
+//   k_dt_reduce          ensembles: each member's minima and TimeIncrement
+//
+// On the structured brick k_nodal_brick (column walks) or k_nodal_block (small
+// bricks) take the place of k_force and k_node, and k_kin_brick (column walks) or
+// k_kin_flat (bricks of up to kKinFlatMax elements an edge) that of k_kin.
 //
 // The Policy template parameter selects the arithmetic of each part:
 // PolicyFp64 keeps everything in FP64 with the reference's association order,
@@ -173,15 +179,15 @@ struct FastDiv {
 
 // Structured-brick description: s elements per edge, lattice node/element
 // numbering of lulesh-init.cc:217-267.  Set when the mesh is the reference's
-// brick, which lets the nodal pass run as one fused kernel.
+// brick, which lets the nodal pass run as one fused kernel.  The k_kin_brick
+// tiles of one problem are 16 x 16.
 struct Brick {
    int32_t s, en;          // elements and nodes per edge
    int32_t tilesX, tilesY; // k_nodal_brick column tiles of (tileW-1) x (rows-1) nodes
    int32_t chunkZ, chunks; // node planes per z-chunk, number of chunks
-   int32_t rows;           // thread rows per k_nodal_brick workgroup: 16 (256 threads) or 8
-                           // for one problem; up to 256 / tileW in ensembles
-   int32_t tileW;          // threads per k_nodal_brick row: 16 for one problem; chosen per
-                           // ensemble member (4..64)
+   int32_t rows;           // thread rows per k_nodal_brick workgroup: 16 or 8 of 16 threads,
+                           // or 256 / tileW (ensemble members, pick_brick_walk)
+   int32_t tileW;          // threads per k_nodal_brick row (4..64)
    FastDiv divS, divS2;    // element index -> (a, b, c)
    // k_kin_brick: 16x16-element column tiles per edge, element planes per z-chunk
    int32_t kinTiles, kinChunk, kinChunks;
