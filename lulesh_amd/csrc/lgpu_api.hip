@@ -1005,8 +1005,9 @@ int lgpu_run(lgpu_ctx *c, lgpu_time_state *ts, int32_t maxCycle)
    HIP_OR_RETURN(c, hipGetLastError());
 
    const bool fold = c->s.isBrick
-                        ? c->s.nodalBlock && fold_start(block_blocks(c->s.brick), c->brickSlots)
-                        : fold_start((c->numElem + c->block - 1) / c->block, c->genericSlots);
+                        ? c->s.nodalBlock && fold_start(block_blocks(c->s.brick), c->brickSlots,
+                                                      c->precision != LGPU_MIXED)
+                        : fold_start((c->numElem + c->block - 1) / c->block, c->genericSlots, false);
    // Cycle j reads the time state, error flags and dt slots of set j mod 2 and
    // writes the other set.
    auto use_sets = [&](int j) {

@@ -61,11 +61,16 @@ inline void add_eos_slots(std::vector<EosSlot> &slots, const EosGroup &g, bool s
 
 // Whether a device-loop cycle begins in its first kernel (k_nodal_block or
 // k_force, of `blocks` workgroups on `slots` resident ones) instead of
-// k_begin_cycle, a launch of 3.0 to 4.7 us.  Each workgroup then starts about
-// 1 us later, so the gain is gone after a few rounds.  Launch / first kernel,
-// us a cycle, FP64: s=8 24.6 / 21.5, s=30 25.8 / 24.1, s=45 40.1 / 39.1, s=64
-// gathers (2 rounds) 68.8 / 68.8; k_nodal_brick s=101 4.7 less and 5.5 more.
-inline bool fold_start(int64_t blocks, int64_t slots) { return blocks <= 2 * slots; }
+// k_begin_cycle, a launch of 3.0 to 4.7 us.  Each workgroup then starts up to 1
+// us later, so the gain is gone after a few rounds (4 of k_nodal_block in FP64,
+// otherwise 2).  Launch / first kernel, us a cycle, FP64: s=8 24.6 / 21.5, s=45
+// 37.6 / 36.1, s=55 (2.4 rounds) 46.7 / 45.7, s=64 (3.6) 64.6 / 63.8; FP64_FMA s=64
+// 58.5 / 57.5; mixed s=63 (2.4) 44.5 / 44.9, s=70 (3.4) 52.5 / 55.3; gathers s=64
+// (2) 82.2 / 81.2, s=72 (2.9) 108.6 / 108.3.
+inline bool fold_start(int64_t blocks, int64_t slots, bool fp64Block)
+{
+   return blocks <= (fp64Block ? 4 : 2) * slots;
+}
 
 // EOS repeat count of region r (0-based), lulesh.cc:2390-2400.
 inline int32_t region_rep(int32_t r, int32_t numReg, int32_t cost)
