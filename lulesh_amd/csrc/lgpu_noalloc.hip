@@ -22,6 +22,10 @@ namespace {
 constexpr int kNaBlock = 256;       // threads per workgroup
 constexpr int kNaMaxBlocks = 2048;  // workgroups of the partial kernel (grid-stride beyond)
 constexpr int kNaMaxDevices = 64;
+// Lists of up to this many elements take one workgroup of 1,024 threads and one
+// launch.  Two launches / one, call and wait, us: 64 elements 17.0 / 14.5, 1,024
+// 16.3 / 14.3, 3,000 16.5 / 15.2 (listed 16.5 / 16.2), 4,096 16.5 / 16.2 (16.6 / 17.4).
+constexpr int kNaSmall = 3072, kNaSmallBlock = 1024;
 
 // Block partials: [2*b] Courant, [2*b+1] hydro.
 __device__ __align__(256) double scratch[2 * kNaMaxBlocks];
@@ -55,9 +59,10 @@ __device__ __forceinline__ double na_wave_min(double v)
 }
 
 // Block minimum of (a, b), valid in thread 0.
+template <int BLOCK>
 __device__ __forceinline__ void na_block_min2(double &a, double &b)
 {
-   __shared__ double sa[kNaBlock / 64], sb[kNaBlock / 64];
+   __shared__ double sa[BLOCK / 64], sb[BLOCK / 64];
    a = na_wave_min(a);
    b = na_wave_min(b);
    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -67,7 +72,7 @@ __device__ __forceinline__ void na_block_min2(double &a, double &b)
    }
    __syncthreads();
    if (threadIdx.x == 0)
-      for (int i = 1; i < kNaBlock / 64; ++i) {
+      for (int i = 1; i < BLOCK / 64; ++i) {
          a = (sa[i] < a) ? sa[i] : a;
          b = (sb[i] < b) ? sb[i] : b;
       }
@@ -77,14 +82,17 @@ __device__ __forceinline__ void na_block_min2(double &a, double &b)
 // of the listed elements, min-reduced per workgroup into part[2*blockIdx].
 // Candidates are taken only where vdov != 0, as in the reference; the
 // minimum does not depend on the order of the elements.
-__global__ void __launch_bounds__(kNaBlock)
+// BLOCK threads per workgroup; the small lists' only workgroup gives the result
+// itself.
+template <int BLOCK>
+__global__ void __launch_bounds__(BLOCK)
 k_tc_partial(const double *__restrict__ ss, const double *__restrict__ vdov,
              const double *__restrict__ arealg, const int32_t *__restrict__ list, int32_t n,
              double qqc2, double dvovmax, double *__restrict__ part)
 {
    double dtc = 1.0e+20, dth = 1.0e+20;
-   const int64_t stride = (int64_t)gridDim.x * kNaBlock;
-   for (int64_t i = (int64_t)blockIdx.x * kNaBlock + threadIdx.x; i < n; i += stride) {
+   const int64_t stride = (int64_t)gridDim.x * BLOCK;
+   for (int64_t i = (int64_t)blockIdx.x * BLOCK + threadIdx.x; i < n; i += stride) {
       const int32_t e = list ? list[i] : (int32_t)i;
       const double vd = vdov[e];
       if (vd == 0.) continue;
@@ -98,7 +106,7 @@ k_tc_partial(const double *__restrict__ ss, const double *__restrict__ vdov,
       const double dtdvov = dvovmax / (fabs(vd) + 1.e-20);
       if (dtdvov < dth) dth = dtdvov;
    }
-   na_block_min2(dtc, dth);
+   na_block_min2<BLOCK>(dtc, dth);
    if (threadIdx.x == 0) {
       part[2 * blockIdx.x] = dtc;
       part[2 * blockIdx.x + 1] = dth;
@@ -115,7 +123,7 @@ k_tc_final(const double *__restrict__ part, int nPart, double *__restrict__ out)
       c = (pc < c) ? pc : c;
       h = (ph < h) ? ph : h;
    }
-   na_block_min2(c, h);
+   na_block_min2<kNaBlock>(c, h);
    if (threadIdx.x == 0) {
       out[0] = c;
       out[1] = h;
@@ -141,8 +149,13 @@ extern "C" int lgpu_time_constraints_noalloc(const double *ss, const double *vdo
    const int64_t want = ((int64_t)numElem + kNaBlock - 1) / kNaBlock;
    const int grid = (int)(want < kNaMaxBlocks ? want : kNaMaxBlocks);
    const double qqc2 = 64.0 * qqc * qqc;
+   if (numElem <= kNaSmall) {
+      hipLaunchKernelGGL(k_tc_partial<kNaSmallBlock>, dim3(1), dim3(kNaSmallBlock), 0, st, ss, vdov, arealg,
+                         elemlist, numElem, qqc2, dvovmax, dtOut);
+      return hipGetLastError() == hipSuccess ? LGPU_OK : LGPU_EDEVICE;
+   }
    if (grid > 0)
-      hipLaunchKernelGGL(k_tc_partial, dim3(grid), dim3(kNaBlock), 0, st, ss, vdov, arealg,
+      hipLaunchKernelGGL(k_tc_partial<kNaBlock>, dim3(grid), dim3(kNaBlock), 0, st, ss, vdov, arealg,
                          elemlist, numElem, qqc2, dvovmax, part);
    hipLaunchKernelGGL(k_tc_final, dim3(1), dim3(kNaBlock), 0, st, part, grid, dtOut);
    if (hipGetLastError() != hipSuccess) return LGPU_EDEVICE;
