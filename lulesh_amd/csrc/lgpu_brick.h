@@ -124,14 +124,19 @@ inline WalkTime walk_time(int64_t columns, int planes, int slots, int chunk, dou
 }
 
 // Time of the fused nodal kernel's walk in planes.  The last chunks that run
-// beyond the others have a CU's units to themselves and count half.  FP64,
-// chunk by rounds of equal chunks / by this, us: s=90 10 / 9, 82 / 75; s=101
-// 11 / 10, 88 / 82; s=128 22 / 21, 180 / 173; s=160 41 / 39, 327 / 311; s=192
-// 65 / 64, 511 / 505; s=200 41 / 39, 635 / 611.
+// beyond the others have a CU's units to themselves and count half; those of at
+// most a quarter of a walk fit into the spread of the others' ends and count a
+// quarter (s=185 chunk 60 to 58, last walk 7 to 13 of 59: 487 / 479 us; 56, 19 of
+// 57: 481).  FP64, chunk by rounds of equal chunks / by this, us: s=90 10 / 9, 82 /
+// 75; s=101 11 / 10, 88 / 82; s=128 22 / 21, 180 / 173; s=160 41 / 39, 327 / 311;
+// s=192 65 / 60, 511 / 488; s=200 41 / 39, 635 / 611.  With all last walks at half
+// / short ones at a quarter: s=113 124 / 117, 120 150 / 144, 185 492 / 479, 192
+// 505 / 488 (FP64_FMA 428 / 413), 202 629 / 617, 243 1095 / 1034, 250 1137 / 1070.
 inline double walk_cost(int64_t columns, int planes, int slots, int chunk)
 {
    const WalkTime t = walk_time(columns, planes, slots, chunk, 1.0);
-   return 0.5 * (t.whole + t.end);
+   const bool shortLast = 4 * (planes % chunk + 1) <= chunk + 1;
+   return t.whole + (shortLast ? 0.25 : 0.5) * (t.end - t.whole);
 }
 
 // Default node planes per workgroup of the fused nodal kernel (at least
