@@ -49,6 +49,12 @@ __global__ void k_time_increment_ens(EnsTime t, const double *dtOut, const int32
    time_increment(t, m, dtOut[2 * m], dtOut[2 * m + 1], any_error(err + m * kNumErrSites));
 }
 
+// The brick path's kernels and the z-chunks of those that walk up columns.
+struct BrickChoice {
+   int nodalChunk = 8, kinChunk = 12;
+   int32_t nodalBlock = 0, kinFlat = 0;
+};
+
 } // namespace
 
 struct lgpu_ensemble {
@@ -76,10 +82,9 @@ struct lgpu_ensemble {
    hipGraph_t graph2 = nullptr;
    hipGraphExec_t exec2 = nullptr;
    std::vector<int32_t> memberSize;
-   int nodalChunk = 8, kinChunk = 12;
+   BrickChoice choice; // what s and the tables are made for
    unsigned nodalBlocks = 0, kinBlocks = 0;
    char *tables = nullptr;
-   size_t tablesBytes = 0;
    int64_t kLaunches[kENumKernels] = {};
    double kMs[kENumKernels] = {};
    std::string lastError;
@@ -246,8 +251,9 @@ int launch_graph(lgpu_ensemble *e)
 // over all members' workgroups.  30 members of 10..40: a walk, 68.7 us
 // (k_nodal_block 84.8); 24 of 5..24: k_nodal_block, FP64 18.6 and mixed 13.6
 // us (best walk 24.1 and 18.5).
-void pick_brick_kernels(lgpu_ensemble *e)
+BrickChoice pick_brick_kernels(const lgpu_ensemble *e)
 {
+   BrickChoice pick;
    int dev = 0, cus = 0, perCu = 0, largest = 0;
    if (hipGetDevice(&dev) != hipSuccess ||
        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
@@ -268,22 +274,23 @@ void pick_brick_kernels(lgpu_ensemble *e)
       largest = std::max(largest, sz);
       bricks.push_back(g);
    }
-   e->s.kinFlat = largest <= kKinFlatMax;
-   if (slots < 1) return;
+   pick.kinFlat = largest <= kKinFlatMax;
+   if (slots < 1) return pick;
    std::vector<int64_t> columns;
    std::vector<int> planes;
    for (const Brick &g : bricks) {
       columns.push_back((int64_t)g.tilesX * g.tilesY);
       planes.push_back(g.en);
    }
-   e->nodalChunk = pick_tail_chunk(columns, planes, slots, 0.25, e->nodalChunk);
+   pick.nodalChunk = pick_tail_chunk(columns, planes, slots, 0.25, pick.nodalChunk);
    double least = 1e300;
    for (int ch = 1; ch <= 22; ++ch) {
       int64_t walks = 0;
       for (const Brick &g : bricks) walks += (int64_t)g.tilesX * g.tilesY * ((g.en + ch - 1) / ch);
       least = std::min(least, (double)((walks + slots - 1) / slots * (ch + 1)));
    }
-   e->s.nodalBlock = block_is_faster(blocks, slots, least);
+   pick.nodalBlock = block_is_faster(blocks, slots, least);
+   return pick;
 }
 
 // The workgroups of a walking kernel over all members: those of whole z-chunks
@@ -348,9 +355,10 @@ void order_eos_blocks(std::vector<EosSlot> &slots, std::vector<EosBlock> &blocks
    blocks.swap(b2);
 }
 
-// Member tables of the brick path for the current kernel and chunk choices:
-// per-member bricks with offsets, and the kernels' workgroups.
-int build_brick_tables(lgpu_ensemble *e)
+// Takes the kernels and chunks of `want`, with the member tables for them:
+// per-member bricks with offsets, and the kernels' workgroups.  Where it fails,
+// the ensemble keeps those it has.
+int set_brick_choice(lgpu_ensemble *e, const BrickChoice &want)
 {
    const int M = e->nMembers;
    std::vector<MemberBrick> mb((size_t)M);
@@ -362,41 +370,48 @@ int build_brick_tables(lgpu_ensemble *e)
       init_brick(g, e->memberSize[(size_t)m]);
       pick_member_tile(g);
       pick_member_kin_tile(g);
-      set_brick_chunk(g, e->nodalChunk);
-      set_kin_chunk(g, e->kinChunk);
+      set_brick_chunk(g, want.nodalChunk);
+      set_kin_chunk(g, want.kinChunk);
       mb[(size_t)m].g = g;
       mb[(size_t)m].nodeOff = e->nodeStart[(size_t)m];
       mb[(size_t)m].elemOff = e->elemStart[(size_t)m];
-      nodalCount.push_back(e->s.nodalBlock ? block_blocks(g) : (int64_t)g.tilesX * g.tilesY);
-      kinCount.push_back(e->s.kinFlat ? flat_blocks(g) : (int64_t)g.kinTilesX * g.kinTilesY);
+      nodalCount.push_back(want.nodalBlock ? block_blocks(g) : (int64_t)g.tilesX * g.tilesY);
+      kinCount.push_back(want.kinFlat ? flat_blocks(g) : (int64_t)g.kinTilesX * g.kinTilesY);
       nodePlanes.push_back(g.en);
       elemPlanes.push_back(g.s);
    }
-   e->s.nodalWhole = e->s.nodalBlock ? equal_blocks(nodalCount, nodal)
-                                     : walk_blocks(nodalCount, nodePlanes, e->nodalChunk, nodal);
-   e->s.kinWhole = e->s.kinFlat ? equal_blocks(kinCount, kin)
-                                : walk_blocks(kinCount, elemPlanes, e->kinChunk, kin);
+   const int32_t nodalWhole = want.nodalBlock ? equal_blocks(nodalCount, nodal)
+                                              : walk_blocks(nodalCount, nodePlanes, want.nodalChunk, nodal);
+   const int32_t kinWhole = want.kinFlat ? equal_blocks(kinCount, kin)
+                                         : walk_blocks(kinCount, elemPlanes, want.kinChunk, kin);
    const size_t nb = nodal.size(), kb = kin.size();
    const size_t b0 = align_up(sizeof(MemberBrick) * (size_t)M);
    const size_t b1 = align_up(sizeof(MemberBlock) * nb), b2 = align_up(sizeof(MemberBlock) * kb);
-   const size_t need = b0 + b1 + b2;
-   ENS_HIP(e, hipStreamSynchronize(e->stream));
-   if (need > e->tablesBytes) {
-      if (e->tables) ENS_HIP(e, hipFree(e->tables));
-      e->tables = nullptr;
-      e->tablesBytes = 0;
-      ENS_HIP(e, hipMalloc((void **)&e->tables, need));
-      e->tablesBytes = need;
+   char *tables = nullptr;
+   ENS_HIP(e, hipMalloc((void **)&tables, b0 + b1 + b2));
+   hipError_t err = hipMemcpy(tables, mb.data(), sizeof(MemberBrick) * (size_t)M, hipMemcpyHostToDevice);
+   if (err == hipSuccess)
+      err = hipMemcpy(tables + b0, nodal.data(), sizeof(MemberBlock) * nb, hipMemcpyHostToDevice);
+   if (err == hipSuccess)
+      err = hipMemcpy(tables + b0 + b1, kin.data(), sizeof(MemberBlock) * kb, hipMemcpyHostToDevice);
+   if (err == hipSuccess) err = hipStreamSynchronize(e->stream); // nothing reads the old ones any more
+   if (err != hipSuccess) {
+      (void)hipFree(tables);
+      return fail_hip(e, err, "brick tables");
    }
-   ENS_HIP(e, hipMemcpy(e->tables, mb.data(), sizeof(MemberBrick) * (size_t)M, hipMemcpyHostToDevice));
-   ENS_HIP(e, hipMemcpy(e->tables + b0, nodal.data(), sizeof(MemberBlock) * nb, hipMemcpyHostToDevice));
-   ENS_HIP(e, hipMemcpy(e->tables + b0 + b1, kin.data(), sizeof(MemberBlock) * kb, hipMemcpyHostToDevice));
-   e->s.memberBrick = reinterpret_cast<const MemberBrick *>(e->tables);
-   e->s.nodalBlocks = reinterpret_cast<const MemberBlock *>(e->tables + b0);
-   e->s.kinBlocks = reinterpret_cast<const MemberBlock *>(e->tables + b0 + b1);
+   drop_graph(e);
+   if (e->tables) (void)hipFree(e->tables);
+   e->tables = tables;
+   e->choice = want;
+   e->s.nodalBlock = want.nodalBlock;
+   e->s.kinFlat = want.kinFlat;
+   e->s.nodalWhole = nodalWhole;
+   e->s.kinWhole = kinWhole;
+   e->s.memberBrick = reinterpret_cast<const MemberBrick *>(tables);
+   e->s.nodalBlocks = reinterpret_cast<const MemberBlock *>(tables + b0);
+   e->s.kinBlocks = reinterpret_cast<const MemberBlock *>(tables + b0 + b1);
    e->nodalBlocks = (unsigned)nb;
    e->kinBlocks = (unsigned)kb;
-   drop_graph(e);
    return LGPU_OK;
 }
 
@@ -706,8 +721,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
              h2d((void *)s.memberBlockStart, blockStart.data(), 4 * blockStart.size()) &&
              h2d(s.v, ones.data(), 8 * E);
    if (!ok) return bail(LGPU_EDEVICE);
-   if (e->brick) pick_brick_kernels(e);
-   if (e->brick && build_brick_tables(e) != LGPU_OK) return bail(LGPU_EDEVICE);
+   if (e->brick && set_brick_choice(e, pick_brick_kernels(e)) != LGPU_OK) return bail(LGPU_EDEVICE);
    if (copies_by_kernel(e->nodeCount, e->elemCount, kSmallMembers, prec == LGPU_MIXED))
       e->small.limit = kSmallMembers;
    if (hipHostMalloc((void **)&e->host, small_copy_bytes(e->small.limit) + (size_t)nMembers * (9 * 8 + 8) + 64 +
@@ -925,17 +939,19 @@ int lgpu_ensemble_set_option(lgpu_ensemble *e, int option, int64_t value)
       drop_graph(e);
       return LGPU_OK;
    case LGPU_ENS_OPT_BRICK_CHUNK:
-   case LGPU_ENS_OPT_KIN_CHUNK:
+   case LGPU_ENS_OPT_KIN_CHUNK: {
       if (!e->brick || value < 1 || value > 1024) return LGPU_EINVAL;
       // a chunk asks for the kernel that walks up columns
+      BrickChoice want = e->choice;
       if (option == LGPU_ENS_OPT_BRICK_CHUNK) {
-         e->nodalChunk = (int)value;
-         e->s.nodalBlock = 0;
+         want.nodalChunk = (int)value;
+         want.nodalBlock = 0;
       } else {
-         e->kinChunk = (int)value;
-         e->s.kinFlat = 0;
+         want.kinChunk = (int)value;
+         want.kinFlat = 0;
       }
-      return build_brick_tables(e);
+      return set_brick_choice(e, want);
+   }
    default:
       return LGPU_EINVAL;
    }
@@ -953,11 +969,11 @@ int lgpu_ensemble_get_option(lgpu_ensemble *e, int option, int64_t *value)
    case LGPU_ENS_OPT_XCD_REMAP: *value = e->s.xcdRemap; return LGPU_OK;
    case LGPU_ENS_OPT_BRICK_CHUNK:
       if (!e->brick) return LGPU_EINVAL;
-      *value = e->nodalChunk;
+      *value = e->choice.nodalChunk;
       return LGPU_OK;
    case LGPU_ENS_OPT_KIN_CHUNK:
       if (!e->brick) return LGPU_EINVAL;
-      *value = e->kinChunk;
+      *value = e->choice.kinChunk;
       return LGPU_OK;
    case LGPU_ENS_OPT_PATH: *value = e->brick ? 1 : 0; return LGPU_OK;
    default: return LGPU_EINVAL;
@@ -999,44 +1015,40 @@ int lgpu_ensemble_autotune(lgpu_ensemble *e, const lgpu_time_state *ts, int32_t 
       // k_nodal_block and k_kin_flat (candidate 0) and the chunks of the
       // walking kernels, then the XCD mapping.
       const int nodalCands[] = {0, 2, 4, 6, 8, 11, 16, 22}, kinCands[] = {0, 4, 6, 8, 12, 16};
-      float best = 1e30f;
-      int bestC = e->nodalChunk;
-      auto set_nodal = [&](int c) {
-         e->s.nodalBlock = c == 0;
-         if (c) e->nodalChunk = c;
-      };
-      auto set_kin = [&](int c) {
-         e->s.kinFlat = c == 0;
-         if (c) e->kinChunk = c;
-      };
+      const BrickChoice before = e->choice;
+      BrickChoice best = before;
+      float bestMs = 1e30f;
       for (int c : nodalCands) {
-         set_nodal(c);
-         r = build_brick_tables(e);
+         BrickChoice want = before;
+         want.nodalBlock = c == 0;
+         if (c) want.nodalChunk = c;
+         r = set_brick_choice(e, want);
          float ms[kENumKernels];
          if (!r) r = trial(ms);
          if (r) break;
-         if (ms[kENodalBrick] < best) {
-            best = ms[kENodalBrick];
-            bestC = c;
+         if (ms[kENodalBrick] < bestMs) {
+            bestMs = ms[kENodalBrick];
+            best = want;
          }
       }
-      set_nodal(bestC);
-      best = 1e30f;
-      bestC = e->kinChunk;
+      bestMs = 1e30f;
       for (int c : kinCands) {
          if (r) break;
-         set_kin(c);
-         r = build_brick_tables(e);
+         BrickChoice want = best;
+         want.kinFlat = c == 0;
+         if (c) want.kinChunk = c;
+         r = set_brick_choice(e, want);
          float ms[kENumKernels];
          if (!r) r = trial(ms);
          if (r) break;
-         if (ms[kEKinBrick] < best) {
-            best = ms[kEKinBrick];
-            bestC = c;
+         if (ms[kEKinBrick] < bestMs) {
+            bestMs = ms[kEKinBrick];
+            best.kinFlat = want.kinFlat;
+            best.kinChunk = want.kinChunk;
          }
       }
-      set_kin(bestC);
-      if (!r) r = build_brick_tables(e);
+      if (!r) r = set_brick_choice(e, best);
+      else (void)set_brick_choice(e, before);
    } else {
       // Each of the three launch-shape-sensitive kernels is tuned over the
       // block sizes.
