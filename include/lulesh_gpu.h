@@ -313,12 +313,18 @@ enum lgpu_ensemble_option {
    LGPU_ENS_OPT_BLOCK_KIN = 5,
    LGPU_ENS_OPT_XCD_REMAP = 6,
    LGPU_ENS_OPT_BRICK_CHUNK = 7,  /* brick path: node planes per workgroup of
-                                     the fused nodal kernel, every member;
-                                     selects the kernel that walks up columns */
+                                     the fused nodal kernel that walks up
+                                     columns, every member.  While the small-
+                                     brick kernel is in use, its present value
+                                     stands for that; any other selects the walk */
    LGPU_ENS_OPT_KIN_CHUNK = 8,    /* brick path: element planes per
-                                     workgroup of the kinematics kernel;
-                                     selects the column walk                  */
-   LGPU_ENS_OPT_PATH = 9          /* read only: 1 brick path, 0 CSR gathers   */
+                                     workgroup of the kinematics kernel that
+                                     walks up columns; as above               */
+   LGPU_ENS_OPT_PATH = 9,         /* read only: 1 brick path, 0 CSR gathers   */
+   LGPU_ENS_OPT_NODAL_KERNEL = 10, /* brick path: 1 the small-brick nodal kernel,
+                                     0 the column walk (default: by the members'
+                                     sizes; the autotuner's choice)           */
+   LGPU_ENS_OPT_KIN_KERNEL = 11   /* the same for the kinematics kernel       */
 };
 int lgpu_ensemble_set_option(lgpu_ensemble *ens, int option, int64_t value);
 int lgpu_ensemble_get_option(lgpu_ensemble *ens, int option, int64_t *value);

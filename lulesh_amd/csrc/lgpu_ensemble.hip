@@ -49,10 +49,25 @@ __global__ void k_time_increment_ens(EnsTime t, const double *dtOut, const int32
    time_increment(t, m, dtOut[2 * m], dtOut[2 * m + 1], any_error(err + m * kNumErrSites));
 }
 
-// The brick path's kernels and the z-chunks of those that walk up columns.
+// The brick path's kernels (1: k_nodal_block, k_kin_flat) and the z-chunks of
+// those that walk up columns.  blockChunk, flatChunk: the chunk that stood there
+// when k_nodal_block or k_kin_flat was chosen (0: they were not), so that a
+// chunk option set to what it reads keeps, or brings back, that kernel.
 struct BrickChoice {
    int nodalChunk = 8, kinChunk = 12;
    int32_t nodalBlock = 0, kinFlat = 0;
+   int blockChunk = 0, flatChunk = 0;
+
+   void choose_nodal(bool block)
+   {
+      nodalBlock = block;
+      blockChunk = block ? nodalChunk : 0;
+   }
+   void choose_kin(bool flat)
+   {
+      kinFlat = flat;
+      flatChunk = flat ? kinChunk : 0;
+   }
 };
 
 } // namespace
@@ -274,7 +289,7 @@ BrickChoice pick_brick_kernels(const lgpu_ensemble *e)
       largest = std::max(largest, sz);
       bricks.push_back(g);
    }
-   pick.kinFlat = largest <= kKinFlatMax;
+   pick.choose_kin(largest <= kKinFlatMax);
    if (slots < 1) return pick;
    std::vector<int64_t> columns;
    std::vector<int> planes;
@@ -289,7 +304,7 @@ BrickChoice pick_brick_kernels(const lgpu_ensemble *e)
       for (const Brick &g : bricks) walks += (int64_t)g.tilesX * g.tilesY * ((g.en + ch - 1) / ch);
       least = std::min(least, (double)((walks + slots - 1) / slots * (ch + 1)));
    }
-   pick.nodalBlock = block_is_faster(blocks, slots, least);
+   pick.choose_nodal(block_is_faster(blocks, slots, least));
    return pick;
 }
 
@@ -941,15 +956,22 @@ int lgpu_ensemble_set_option(lgpu_ensemble *e, int option, int64_t value)
    case LGPU_ENS_OPT_BRICK_CHUNK:
    case LGPU_ENS_OPT_KIN_CHUNK: {
       if (!e->brick || value < 1 || value > 1024) return LGPU_EINVAL;
-      // a chunk asks for the kernel that walks up columns
       BrickChoice want = e->choice;
       if (option == LGPU_ENS_OPT_BRICK_CHUNK) {
          want.nodalChunk = (int)value;
-         want.nodalBlock = 0;
+         want.nodalBlock = want.nodalChunk == want.blockChunk;
       } else {
          want.kinChunk = (int)value;
-         want.kinFlat = 0;
+         want.kinFlat = want.kinChunk == want.flatChunk;
       }
+      return set_brick_choice(e, want);
+   }
+   case LGPU_ENS_OPT_NODAL_KERNEL:
+   case LGPU_ENS_OPT_KIN_KERNEL: {
+      if (!e->brick || (value != 0 && value != 1)) return LGPU_EINVAL;
+      BrickChoice want = e->choice;
+      if (option == LGPU_ENS_OPT_NODAL_KERNEL) want.choose_nodal(value == 1);
+      else want.choose_kin(value == 1);
       return set_brick_choice(e, want);
    }
    default:
@@ -976,6 +998,11 @@ int lgpu_ensemble_get_option(lgpu_ensemble *e, int option, int64_t *value)
       *value = e->choice.kinChunk;
       return LGPU_OK;
    case LGPU_ENS_OPT_PATH: *value = e->brick ? 1 : 0; return LGPU_OK;
+   case LGPU_ENS_OPT_NODAL_KERNEL:
+   case LGPU_ENS_OPT_KIN_KERNEL:
+      if (!e->brick) return LGPU_EINVAL;
+      *value = option == LGPU_ENS_OPT_NODAL_KERNEL ? e->choice.nodalBlock : e->choice.kinFlat;
+      return LGPU_OK;
    default: return LGPU_EINVAL;
    }
 }
@@ -1012,41 +1039,48 @@ int lgpu_ensemble_autotune(lgpu_ensemble *e, const lgpu_time_state *ts, int32_t 
    };
    int r = LGPU_OK;
    if (e->brick) {
-      // k_nodal_block and k_kin_flat (candidate 0) and the chunks of the
-      // walking kernels, then the XCD mapping.
-      const int nodalCands[] = {0, 2, 4, 6, 8, 11, 16, 22}, kinCands[] = {0, 4, 6, 8, 12, 16};
+      // The chunks of the walking kernels, with k_nodal_block and k_kin_flat
+      // against the best of them, then the XCD mapping.
+      const int nodalCands[] = {4, 6, 8, 11, 16, 22}, kinCands[] = {4, 6, 8, 12, 16};
       const BrickChoice before = e->choice;
       BrickChoice best = before;
-      float bestMs = 1e30f;
-      for (int c : nodalCands) {
-         BrickChoice want = before;
-         want.nodalBlock = c == 0;
-         if (c) want.nodalChunk = c;
-         r = set_brick_choice(e, want);
+      auto time_choice = [&](const BrickChoice &want, int kernel, float &t) {
          float ms[kENumKernels];
-         if (!r) r = trial(ms);
+         int st = set_brick_choice(e, want);
+         if (!st) st = trial(ms);
+         t = st ? 1e30f : ms[kernel];
+         return st;
+      };
+      float bestMs = 1e30f, t = 0.f;
+      for (int c : nodalCands) {
          if (r) break;
-         if (ms[kENodalBrick] < bestMs) {
-            bestMs = ms[kENodalBrick];
-            best = want;
+         BrickChoice want = best;
+         want.nodalChunk = c;
+         want.choose_nodal(false);
+         r = time_choice(want, kENodalBrick, t);
+         if (!r && t < bestMs) {
+            bestMs = t;
+            best.nodalChunk = c;
          }
       }
+      best.choose_nodal(true);
+      if (!r) r = time_choice(best, kENodalBrick, t);
+      best.choose_nodal(t <= bestMs);
       bestMs = 1e30f;
       for (int c : kinCands) {
          if (r) break;
          BrickChoice want = best;
-         want.kinFlat = c == 0;
-         if (c) want.kinChunk = c;
-         r = set_brick_choice(e, want);
-         float ms[kENumKernels];
-         if (!r) r = trial(ms);
-         if (r) break;
-         if (ms[kEKinBrick] < bestMs) {
-            bestMs = ms[kEKinBrick];
-            best.kinFlat = want.kinFlat;
-            best.kinChunk = want.kinChunk;
+         want.kinChunk = c;
+         want.choose_kin(false);
+         r = time_choice(want, kEKinBrick, t);
+         if (!r && t < bestMs) {
+            bestMs = t;
+            best.kinChunk = c;
          }
       }
+      best.choose_kin(true);
+      if (!r) r = time_choice(best, kEKinBrick, t);
+      best.choose_kin(t <= bestMs);
       if (!r) r = set_brick_choice(e, best);
       else (void)set_brick_choice(e, before);
    } else {

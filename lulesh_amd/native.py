@@ -482,7 +482,8 @@ def ensemble_draw(n: int, seed: int = 1234):
 
 
 ENS_OPT_GRAPH, ENS_OPT_TIMING, ENS_OPT_BLOCK_FORCE, ENS_OPT_BLOCK_NODE, ENS_OPT_BLOCK_KIN, \
-    ENS_OPT_XCD_REMAP, ENS_OPT_BRICK_CHUNK, ENS_OPT_KIN_CHUNK, ENS_OPT_PATH = 1, 2, 3, 4, 5, 6, 7, 8, 9
+    ENS_OPT_XCD_REMAP, ENS_OPT_BRICK_CHUNK, ENS_OPT_KIN_CHUNK, ENS_OPT_PATH, ENS_OPT_NODAL_KERNEL, \
+    ENS_OPT_KIN_KERNEL = 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11
 
 
 class Ensemble:
@@ -559,6 +560,8 @@ class Ensemble:
         if self.brick:
             return {"path": "brick", "brick_chunk": self.get_option(ENS_OPT_BRICK_CHUNK),
                     "kin_chunk": self.get_option(ENS_OPT_KIN_CHUNK),
+                    "nodal_kernel": self.get_option(ENS_OPT_NODAL_KERNEL),
+                    "kin_kernel": self.get_option(ENS_OPT_KIN_KERNEL),
                     "xcd_remap": self.get_option(ENS_OPT_XCD_REMAP)}
         return {"path": "generic", "block_force": self.get_option(ENS_OPT_BLOCK_FORCE),
                 "block_node": self.get_option(ENS_OPT_BLOCK_NODE),
