@@ -225,21 +225,23 @@ enum lgpu_option {
                                      kernels of the generic path: 64, 128
                                      or 256                                  */
    LGPU_OPT_BRICK_CHUNK = 4,      /* node planes per workgroup of the fused
-                                     brick kernel (1..mesh edge); setting it
-                                     selects the kernel that walks up columns,
-                                     also where a small brick has another     */
+                                     brick kernel that walks up columns (1..
+                                     mesh edge).  Small bricks have another
+                                     kernel by default: there the default chunk
+                                     stands for it, any other selects the walk */
    LGPU_OPT_XCD_REMAP = 5,        /* 1 (default): contiguous block ranges per
                                      XCD; 0: hardware order                 */
    LGPU_OPT_KERNEL_TIMING_MASK = 6, /* bit k: time kernel k while timing is on
                                      (default: all)                          */
    LGPU_OPT_KIN_CHUNK = 7,        /* element planes per workgroup of the
-                                     brick kinematics kernel (1..mesh edge);
-                                     setting it selects the column walk       */
+                                     brick kinematics kernel that walks up
+                                     columns (1..mesh edge); small bricks as
+                                     above                                    */
    LGPU_OPT_BRICK_ROWS = 8,       /* thread rows of a fused brick workgroup:
-                                     16 (16x16 element columns, or by default
+                                     16 (default: 16x16 element columns, or
                                      another shape of 256 threads where it
-                                     covers the mesh with fewer) or 8 (16x8);
-                                     setting it selects the column walk       */
+                                     covers the mesh with fewer) or 8 (16x8,
+                                     always the column walk)                  */
    LGPU_OPT_EOS_INTERLEAVE = 9    /* k_eos dispatch order: 0 work-list order,
                                      largest EOS repeat count first; k > 0 one
                                      workgroup of the largest count every k+1

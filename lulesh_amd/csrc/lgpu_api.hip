@@ -63,6 +63,9 @@ struct lgpu_ctx {
    std::vector<PlacedSlot> eosSlots; // in work-list order
    int eosInterleave = 0;
    int32_t brickPerCu = 0;
+   // the default tile, and the chunks that the options read while k_nodal_block
+   // and k_kin_flat are in use (0: not the default kernels of this size)
+   int tileW = 16, tileRows = 16, blockChunk = 0, flatChunk = 0;
    // resident workgroups: nodal brick kernels, k_force, k_eos
    int64_t brickSlots = 0, genericSlots = 0, eosResident = 0;
    bool timing = false;
@@ -271,6 +274,20 @@ int default_interleave(const lgpu_ctx *c)
    while (heavy < all && c->eosSlots[(size_t)heavy].slot.rep == c->eosSlots[0].slot.rep) ++heavy;
    return 5 * heavy > all ? 2 : 4;
 }
+
+// The kernels that the brick options ask for.  The default number of rows
+// stands for the default tile, and the default chunk, where that is a small
+// brick's, for its kernel: an option set to what it reads changes nothing.
+void set_nodal_kernel(lgpu_ctx *c, int rows)
+{
+   Brick &g = c->s.brick;
+   if (rows == 8) set_brick_tile(g, 16, 8);
+   else set_brick_tile(g, c->tileW, c->tileRows);
+   c->s.nodalBlock = rows == 16 && g.chunkZ == c->blockChunk;
+}
+
+// Thread rows as the option gives them: 16 for every tile of 256 threads.
+int option_rows(const lgpu_ctx *c) { return other_tile(c->s.brick) ? 16 : c->s.brick.rows; }
 
 // Device array of a field.  `narrow`: stored as FP32 in the mixed form (the
 // Q gradients, p, q and ss).
@@ -529,6 +546,10 @@ int alloc_context(const CtxSpec &sp, lgpu_ctx **out)
       default: kinPerCu = Launch<PolicyFp64>::kin_brick_blocks_per_cu(); break;
       }
       set_kin_chunk(g, pick_kin_chunk(g, cus * kinPerCu));
+      c->tileW = g.tileW;
+      c->tileRows = g.rows;
+      c->blockChunk = s.nodalBlock ? g.chunkZ : 0;
+      c->flatChunk = s.kinFlat ? g.kinChunk : 0;
    }
    *out = c;
    return LGPU_OK;
@@ -1101,7 +1122,7 @@ int lgpu_set_option(lgpu_ctx *c, int option, int64_t value)
    case LGPU_OPT_BRICK_CHUNK:
       if (!c->s.isBrick || value < 1) return LGPU_EINVAL;
       set_brick_chunk(c->s.brick, (int)std::min<int64_t>(value, 1 << 20));
-      c->s.nodalBlock = 0;
+      set_nodal_kernel(c, option_rows(c));
       return LGPU_OK;
    case LGPU_OPT_XCD_REMAP:
       c->s.xcdRemap = value ? 1 : 0;
@@ -1109,12 +1130,11 @@ int lgpu_set_option(lgpu_ctx *c, int option, int64_t value)
    case LGPU_OPT_KIN_CHUNK:
       if (!c->s.isBrick || value < 1) return LGPU_EINVAL;
       set_kin_chunk(c->s.brick, (int)std::min<int64_t>(value, 1 << 20));
-      c->s.kinFlat = 0;
+      c->s.kinFlat = c->s.brick.kinChunk == c->flatChunk;
       return LGPU_OK;
    case LGPU_OPT_BRICK_ROWS:
       if (!c->s.isBrick || (value != 8 && value != 16)) return LGPU_EINVAL;
-      set_brick_tile(c->s.brick, 16, (int)value);
-      c->s.nodalBlock = 0;
+      set_nodal_kernel(c, (int)value);
       return LGPU_OK;
    case LGPU_OPT_EOS_INTERLEAVE:
       if (value < 0 || value > 1024) return LGPU_EINVAL;
@@ -1146,7 +1166,7 @@ int lgpu_get_option(lgpu_ctx *c, int option, int64_t *value)
       return LGPU_OK;
    case LGPU_OPT_BRICK_ROWS:
       if (!c->s.isBrick) return LGPU_EINVAL;
-      *value = other_tile(c->s.brick) ? 16 : c->s.brick.rows;
+      *value = option_rows(c);
       return LGPU_OK;
    case LGPU_OPT_EOS_INTERLEAVE: *value = c->eosInterleave; return LGPU_OK;
    default: return LGPU_EINVAL;
