@@ -160,52 +160,64 @@ void enqueue_cycle(lgpu_ensemble *e)
    }
 }
 
-// Per-kernel timing of one cycle (used by the autotuner and the timing
-// option): events around each launch.
-template <class P>
-int timed_cycle(lgpu_ensemble *e, float ms[kENumKernels])
-{
-   hipEvent_t ev[kENumKernels + 1];
-   for (auto &x : ev) ENS_HIP(e, hipEventCreate(&x));
-   ENS_HIP(e, hipEventRecord(ev[0], e->stream));
-   ENS_HIP(e, hipEventRecord(ev[1], e->stream));
-   if (e->brick) {
-      Launch<P>::nodal_brick_members(e->s, e->k, e->nodalBlocks, e->stream);
-      swap_nodes(e);
-      ENS_HIP(e, hipEventRecord(ev[2], e->stream));
-      ENS_HIP(e, hipEventRecord(ev[3], e->stream));
-      Launch<P>::kin_brick_members(e->s, e->k, e->kinBlocks, e->stream);
-   } else {
-      Launch<P>::force(e->s, e->k, e->planeStride, e->block[0], e->stream);
-      ENS_HIP(e, hipEventRecord(ev[2], e->stream));
-      Launch<P>::node(e->s, e->k, e->planeStride, 0.0, e->block[1], e->stream);
-      ENS_HIP(e, hipEventRecord(ev[3], e->stream));
-      Launch<P>::kin(e->s, e->k, 0.0, e->block[2], e->stream);
+// Events around launches; the stream is waited for before they are read.
+template <int N>
+struct Events {
+   hipEvent_t ev[N] = {};
+   ~Events()
+   {
+      for (hipEvent_t x : ev)
+         if (x) (void)hipEventDestroy(x);
    }
-   ENS_HIP(e, hipEventRecord(ev[4], e->stream));
-   Launch<P>::eos(e->s, e->k, e->stream);
-   ENS_HIP(e, hipEventRecord(ev[5], e->stream));
-   Launch<P>::dt_reduce(e->s, e->stream);
-   ENS_HIP(e, hipEventRecord(ev[6], e->stream));
+};
+
+void count_launch(lgpu_ensemble *e, int kernel, float ms)
+{
+   e->kLaunches[kernel] += 1;
+   e->kMs[kernel] += ms;
+}
+
+// One cycle with every kernel timed (the timing option; the autotuner).
+template <class P>
+int timed_cycle(lgpu_ensemble *e)
+{
+   std::vector<int> kernels{kEForce, kENode, kEKin, kEEos, kEDt};
+   if (e->brick) kernels = {kENodalBrick, kEKinBrick, kEEos, kEDt};
+   Events<6> events;
+   for (auto &x : events.ev) ENS_HIP(e, hipEventCreate(&x));
+   hipEvent_t *next = events.ev;
+   ENS_HIP(e, hipEventRecord(*next++, e->stream));
+   for (int kernel : kernels) {
+      switch (kernel) {
+      case kENodalBrick:
+         Launch<P>::nodal_brick_members(e->s, e->k, e->nodalBlocks, e->stream);
+         swap_nodes(e);
+         break;
+      case kEKinBrick: Launch<P>::kin_brick_members(e->s, e->k, e->kinBlocks, e->stream); break;
+      case kEForce: Launch<P>::force(e->s, e->k, e->planeStride, e->block[0], e->stream); break;
+      case kENode: Launch<P>::node(e->s, e->k, e->planeStride, 0.0, e->block[1], e->stream); break;
+      case kEKin: Launch<P>::kin(e->s, e->k, 0.0, e->block[2], e->stream); break;
+      case kEEos: Launch<P>::eos(e->s, e->k, e->stream); break;
+      default: Launch<P>::dt_reduce(e->s, e->stream);
+      }
+      ENS_HIP(e, hipEventRecord(*next++, e->stream));
+   }
    ENS_HIP(e, hipGetLastError());
    ENS_HIP(e, hipStreamSynchronize(e->stream));
-   // ev[i]..ev[i+1] brackets: 0 time, 1 force (brick: nodal), 2 node (brick:
-   // empty), 3 kin, 4 eos, 5 dt
-   const int order[6] = {kETime, e->brick ? kENodalBrick : kEForce, kENode,
-                         e->brick ? kEKinBrick : kEKin, kEEos, kEDt};
-   for (int i = 0; i < kENumKernels; ++i) ms[i] = 0.f;
-   for (int i = 0; i < 6; ++i) ENS_HIP(e, hipEventElapsedTime(&ms[order[i]], ev[i], ev[i + 1]));
-   if (e->brick) ms[kENode] = 0.f;
-   for (auto &x : ev) (void)hipEventDestroy(x);
+   for (size_t i = 0; i < kernels.size(); ++i) {
+      float ms = 0.f;
+      ENS_HIP(e, hipEventElapsedTime(&ms, events.ev[i], events.ev[i + 1]));
+      count_launch(e, kernels[i], ms);
+   }
    return LGPU_OK;
 }
 
-int timed_cycle_any(lgpu_ensemble *e, float ms[kENumKernels])
+int timed_cycle_any(lgpu_ensemble *e)
 {
    switch (e->precision) {
-   case LGPU_MIXED: return timed_cycle<PolicyMixed>(e, ms);
-   case LGPU_FP64_FMA: return timed_cycle<PolicyFp64Fma>(e, ms);
-   default: return timed_cycle<PolicyFp64>(e, ms);
+   case LGPU_MIXED: return timed_cycle<PolicyMixed>(e);
+   case LGPU_FP64_FMA: return timed_cycle<PolicyFp64Fma>(e);
+   default: return timed_cycle<PolicyFp64>(e);
    }
 }
 
@@ -865,9 +877,21 @@ int lgpu_ensemble_run(lgpu_ensemble *e, lgpu_time_state *ts, int32_t maxCycle, i
       const int r = build_graph(e);
       if (r) return r;
    }
+   Events<2> start;
+   if (e->timing) {
+      for (auto &x : start.ev) ENS_HIP(e, hipEventCreate(&x));
+      ENS_HIP(e, hipEventRecord(start.ev[0], e->stream));
+   }
    hipLaunchKernelGGL(k_time_increment_ens, dim3((unsigned)((M + 63) / 64)), dim3(64), 0, e->stream,
                       e->t, e->s.memberDtOut, e->s.memberErr, M);
    ENS_HIP(e, hipGetLastError());
+   if (e->timing) {
+      float ms = 0.f;
+      ENS_HIP(e, hipEventRecord(start.ev[1], e->stream));
+      ENS_HIP(e, hipStreamSynchronize(e->stream));
+      ENS_HIP(e, hipEventElapsedTime(&ms, start.ev[0], start.ev[1]));
+      count_launch(e, kETime, ms);
+   }
    // Cycles are enqueued in batches between host checks of the loop flags, and
    // no more of them than the member with the most cycles left can run: only
    // a run that ends at stoptime (or on an error) enqueues no-op cycles.
@@ -879,13 +903,8 @@ int lgpu_ensemble_run(lgpu_ensemble *e, lgpu_time_state *ts, int32_t maxCycle, i
       remaining -= batch;
       for (int b = 0; b < batch; ++b) {
          if (e->timing) {
-            float ms[kENumKernels];
-            const int r = timed_cycle_any(e, ms);
+            const int r = timed_cycle_any(e);
             if (r) return r;
-            for (int i = 0; i < kENumKernels; ++i) {
-               e->kLaunches[i] += 1;
-               e->kMs[i] += ms[i];
-            }
          } else if (e->useGraph) {
             const int r = launch_graph(e);
             if (r) return r;
