@@ -913,7 +913,7 @@ int lgpu_upload(lgpu_ctx *c, int field, const double *host)
       return LGPU_OK;
    }
    HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));
-   if (narrow && (int64_t)n > kConvertOnHost) {
+   if (narrow && converts_on_device(host, (int64_t)n, true)) {
       double *wide = scratch_doubles(c);
       HIP_OR_RETURN(c, hipMemcpy(wide, host, sizeof(double) * n, hipMemcpyHostToDevice));
       HIP_OR_RETURN(c, launch_narrow(wide, reinterpret_cast<float *>(dst), (int64_t)n, c->stream));
@@ -943,7 +943,7 @@ int lgpu_download(lgpu_ctx *c, int field, double *host)
       std::fill(host, host + n, 0.0);
       return LGPU_OK;
    }
-   if (narrow && (int64_t)n > kConvertOnHost) {
+   if (narrow && converts_on_device(host, (int64_t)n, false)) {
       double *wide = scratch_doubles(c);
       HIP_OR_RETURN(c, launch_widen(reinterpret_cast<const float *>(src), wide, (int64_t)n, c->stream));
       HIP_OR_RETURN(c, hipStreamSynchronize(c->stream));

@@ -11,10 +11,14 @@
 
 namespace lgpu {
 
-// Fields of up to this many values are converted on the host, where a launch
-// and its synchronisation cost more than the loop: upload on the host / on the
-// device, 27,000 values 14.8 / 25.4 us, 91,125 34.5 / 34.4, 250,047 69.6 / 56.7.
-constexpr int64_t kConvertOnHost = 98304;
+// Whether a field of n values in the caller's array `host` is converted on the
+// device instead of the host.  Twice the bytes then cross the link, which pinned
+// memory takes at 55 GB/s, but other memory only at the rate of the copy into the
+// runtime's buffers.  Host / device, us: pinned, upload 125,000 values 36.1 / 39.0,
+// 166,375 47.0 / 45.0, 1,000,000 249 / 166, download 103,823 37.4 / 35.2, 1,000,000
+// 362 / 167; not pinned, upload 216,000 62.4 / 85.0, 1,000,000 261 / 249, 2,744,000
+// 832 / 623, download 216,000 74.3 / 121, 1,000,000 376 / 500, 7,077,888 3,797 / 3,695.
+bool converts_on_device(const void *host, int64_t n, bool upload);
 
 // dst[i] = (float)src[i] and dst[i] = src[i] on stream st.  Enqueue only.
 hipError_t launch_narrow(const double *src, float *dst, int64_t n, hipStream_t st);

@@ -99,6 +99,18 @@ hipError_t SmallCopy::download(void *device, double *host, bool fp32, int n, hip
    return w;
 }
 
+bool converts_on_device(const void *host, int64_t n, bool upload)
+{
+   constexpr int64_t kPinnedUp = 150000, kPinnedDown = 98304, kUp = 1 << 20; // converted on the host
+   if (n <= (upload ? kPinnedUp : kPinnedDown)) return false;
+   hipPointerAttribute_t a{};
+   if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+      (void)hipGetLastError(); // memory that the runtime does not know
+      a.type = hipMemoryTypeUnregistered;
+   }
+   return a.type == hipMemoryTypeHost || (upload && n > kUp);
+}
+
 hipError_t launch_narrow(const double *src, float *dst, int64_t n, hipStream_t st)
 {
    return launch(src, dst, n, st);

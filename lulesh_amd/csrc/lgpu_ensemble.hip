@@ -786,7 +786,7 @@ int lgpu_ensemble_upload(lgpu_ensemble *e, int32_t member, int field, const doub
       return LGPU_OK;
    }
    ENS_HIP(e, hipStreamSynchronize(e->stream));
-   if (narrow && (int64_t)n > kConvertOnHost) {
+   if (narrow && converts_on_device(host, (int64_t)n, true)) {
       double *wide = scratch_doubles(e);
       ENS_HIP(e, hipMemcpy(wide, host, 8 * n, hipMemcpyHostToDevice));
       ENS_HIP(e, launch_narrow(wide, static_cast<float *>(dst), (int64_t)n, e->stream));
@@ -815,7 +815,7 @@ int lgpu_ensemble_download(lgpu_ensemble *e, int32_t member, int field, double *
       return LGPU_OK;
    }
    ENS_HIP(e, hipStreamSynchronize(e->stream));
-   if (narrow && (int64_t)n > kConvertOnHost) {
+   if (narrow && converts_on_device(host, (int64_t)n, false)) {
       double *wide = scratch_doubles(e);
       ENS_HIP(e, launch_widen(static_cast<float *>(src), wide, (int64_t)n, e->stream));
       ENS_HIP(e, hipStreamSynchronize(e->stream));

@@ -22,16 +22,17 @@ struct Config {
 
 std::vector<Config> configs;
 std::map<const void *, std::string> kernels; // host stub -> demangled name
-std::map<char *, size_t> live;               // device allocations
+std::map<char *, size_t> live, pinned;       // device allocations, hipHostMalloc
 std::string launches, report;
 long mallocsLeft = -1; // hipMalloc fails once this many have succeeded (< 0: never)
 long copies = 0, capturing = 0;
 
-bool device_pointer(const void *p)
+bool holds(const std::map<char *, size_t> &blocks, const void *p)
 {
-   auto it = live.upper_bound((char *)p);
-   return it != live.begin() && (--it, (const char *)p < it->first + it->second);
+   auto it = blocks.upper_bound((char *)p);
+   return it != blocks.begin() && (--it, (const char *)p < it->first + it->second);
 }
+bool device_pointer(const void *p) { return holds(live, p); }
 
 } // namespace
 
@@ -156,10 +157,18 @@ hipError_t hipFree(void *p)
 hipError_t hipHostMalloc(void **p, size_t bytes, unsigned)
 {
    *p = std::calloc(1, bytes);
+   pinned[(char *)*p] = bytes;
    return hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p)
+{
+   *a = hipPointerAttribute_t{};
+   a->type = holds(pinned, p) ? hipMemoryTypeHost : hipMemoryTypeDevice;
+   return holds(pinned, p) || device_pointer(p) ? hipSuccess : hipErrorInvalidValue;
 }
 hipError_t hipHostFree(void *p)
 {
+   pinned.erase((char *)p);
    std::free(p);
    return hipSuccess;
 }

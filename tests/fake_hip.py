@@ -59,5 +59,10 @@ class Fake:
     def fail_malloc_after(self, n):
         self.lib.fake_fail_malloc_after(n)
 
+    def pinned(self, nbytes):
+        p = ctypes.c_void_p()
+        assert self.lib.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(nbytes), 0) == 0
+        return p
+
     def copies(self):
         return self.lib.fake_copies()
