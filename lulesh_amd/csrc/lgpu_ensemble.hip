@@ -585,6 +585,7 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
    // The EOS work list, as for a single domain: each member's elements grouped
    // by EOS repeat count, largest first, in mesh order within a group.
    std::vector<int32_t> perm, blockStart(1, 0);
+   perm.reserve((size_t)totE);
    std::vector<EosBlock> eosBlock;
    std::vector<EosSlot> eosSlots;
    for (int32_t m = 0; m < nMembers; ++m) {
@@ -596,15 +597,15 @@ int lgpu_ensemble_create(const lgpu_mesh_desc *members, int32_t nMembers, lgpu_e
       e->elemCount.push_back(d.numElem);
       const int32_t e0 = e->elemStart[m];
       std::vector<int32_t> repOf((size_t)d.numElem, 1), reps;
+      double repeats = 0.;
       for (int32_t r = 0; r < d.numReg; ++r) {
          const int32_t rep = region_rep(r, d.numReg, d.cost);
+         repeats += (double)rep * d.regElemSize[r];
          if (d.regElemSize[r] > 0 && std::find(reps.begin(), reps.end(), rep) == reps.end())
             reps.push_back(rep);
          for (int32_t i = 0; i < d.regElemSize[r]; ++i) repOf[(size_t)d.regElemlist[r][i]] = rep;
       }
       std::sort(reps.begin(), reps.end(), std::greater<int32_t>());
-      double repeats = 0.;
-      for (int32_t rep : repOf) repeats += rep;
       for (int32_t rep : reps) {
          const int64_t pos = (int64_t)perm.size();
          for (int32_t el = 0; el < d.numElem; ++el)

@@ -26,6 +26,7 @@ std::map<char *, size_t> live, pinned;       // device allocations, hipHostMallo
 std::string launches, report;
 long mallocsLeft = -1; // hipMalloc fails once this many have succeeded (< 0: never)
 long copies = 0, capturing = 0;
+std::vector<lgpu::EosSlot> eosSlots; // of the last k_eos launch
 
 bool holds(const std::map<char *, size_t> &blocks, const void *p)
 {
@@ -48,6 +49,11 @@ const char *fake_launches()
 }
 void fake_fail_malloc_after(long n) { mallocsLeft = n; }
 long fake_copies() { return copies; } // hipMemcpy calls
+int fake_eos_slots(const lgpu::EosSlot **slots)
+{
+   *slots = eosSlots.data();
+   return (int)eosSlots.size();
+}
 
 // --- registration and launch ---
 void **__hipRegisterFatBinary(const void *)
@@ -110,6 +116,10 @@ hipError_t hipLaunchKernel(const void *host, dim3 grid, dim3 block, void **args,
                }
             }
       }
+   }
+   if (name.find("k_eos<") != std::string::npos) {
+      const lgpu::DevState &s = *static_cast<const lgpu::DevState *>(args[0]);
+      eosSlots.assign(s.eosSlot, s.eosSlot + grid.x);
    }
    launches += name + " " + std::to_string(grid.x) + " " + std::to_string(block.x) + "\n";
    return hipSuccess;

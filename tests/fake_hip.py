@@ -59,6 +59,12 @@ class Fake:
     def fail_malloc_after(self, n):
         self.lib.fake_fail_malloc_after(n)
 
+    def eos_slots(self):
+        """(pos, count, rep, share) of the last k_eos launch's workgroups."""
+        p = ctypes.POINTER(ctypes.c_int32)()
+        n = self.lib.fake_eos_slots(ctypes.byref(p))
+        return [tuple(p[4 * i:4 * i + 4]) for i in range(n)]
+
     def pinned(self, nbytes):
         p = ctypes.c_void_p()
         assert self.lib.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(nbytes), 0) == 0
