@@ -1043,8 +1043,10 @@ int lgpu_run(lgpu_ctx *c, lgpu_time_state *ts, int32_t maxCycle)
       s.active = &s.timeOut->active;
    };
    // The host runs at most kAhead cycles ahead of the last one it has seen
-   // begin, so that the device never waits for it (a check after every 16
-   // cycles left it idle for 13 us).  No more cycles are enqueued than the
+   // begin, so that the device does not wait for it where cycles take less than
+   // the 2 ms that host_reached polls (a check after every 16 cycles left it
+   // idle for 13 us; longer cycles still have one, as the stream is then waited
+   // for).  No more cycles are enqueued than the
    // cycle limit allows, so only a run that ends at stoptime (or on an error)
    // enqueues no-op cycles, at most kAhead.
    constexpr uint32_t kAhead = 16;

@@ -126,12 +126,8 @@ inline WalkTime walk_time(int64_t columns, int planes, int slots, int chunk, dou
 // Time of the fused nodal kernel's walk in planes.  The last chunks that run
 // beyond the others have a CU's units to themselves and count half; those of at
 // most a quarter of a walk fit into the spread of the others' ends and count a
-// quarter (s=185 chunk 60 to 58, last walk 7 to 13 of 59: 487 / 479 us; 56, 19 of
-// 57: 481).  FP64, chunk by rounds of equal chunks / by this, us: s=90 10 / 9, 82 /
-// 75; s=101 11 / 10, 88 / 82; s=128 22 / 21, 180 / 173; s=160 41 / 39, 327 / 311;
-// s=192 65 / 60, 511 / 488; s=200 41 / 39, 635 / 611.  With all last walks at half
-// / short ones at a quarter: s=113 124 / 117, 120 150 / 144, 185 492 / 479, 192
-// 505 / 488 (FP64_FMA 428 / 413), 202 629 / 617, 243 1095 / 1034, 250 1137 / 1070.
+// quarter (FP64 s=192, last walks at half / short ones at a quarter: 505 / 488 us;
+// chunks of equal rounds 511).
 inline double walk_cost(int64_t columns, int planes, int slots, int chunk)
 {
    const WalkTime t = walk_time(columns, planes, slots, chunk, 1.0);
@@ -248,8 +244,7 @@ inline void pick_member_tile(Brick &g)
 inline bool other_tile(const Brick &g) { return g.tileW != 16 || (g.rows != 16 && g.rows != 8); }
 
 // walk_cost of the tile and chunk chosen; a plane takes 7% longer where the
-// tile's width is read at run time (one problem's s=64 FP64: 34.9 us for 20
-// columns in chunks of 3, k_nodal_block 33.5).
+// tile's width is read at run time.
 inline double brick_walk_cost(const Brick &g, int slots)
 {
    if (slots < 1) return 0.;
@@ -260,11 +255,8 @@ inline double brick_walk_cost(const Brick &g, int slots)
 // The fused nodal kernel's tile and chunk for one problem: 16 x 16 threads, or
 // the tile that an ensemble's member of this size would have where that needs
 // 7% fewer columns and the walk is 7% shorter by more than its planes cost.
-// 16 x 16 / that, us, FP64: s=75 54.8 / 49.0, s=90 75.5 / 65.0, s=95 80.3 / 70.2,
-// s=105 112.9 / 100.7, s=120 162 / 152, s=125 171 / 155; FP64_FMA s=90 60.6 / 54.1,
-// s=120 132 / 129; mixed s=75 34.5 / 29.2, s=105 63.5 / 62.5, s=125 126 / 121; not
-// taken: s=84 (35 columns of 36) 54.7 / 56.1, s=110 111.7 / 111.9, FP64_FMA s=140
-// 187 / 196.
+// 16 x 16 / that, us: FP64 s=90 75.5 / 65.0, s=125 171 / 155; not taken: FP64 s=110
+// 111.7 / 111.9, FP64_FMA s=140 187 / 196.
 inline void pick_brick_walk(Brick &g, int slots)
 {
    set_brick_chunk(g, pick_brick_chunk(g, slots, 1));
@@ -336,12 +328,11 @@ inline int64_t block_blocks(const Brick &g) { return (int64_t)g.blkX * g.blkY * 
 
 // True when k_nodal_block is the faster nodal kernel: `blocks` workgroups of
 // it on `slots` resident ones take about 1 + blocks / slots planes of the
-// walking kernel's time (8.3 us a plane in FP64: s=30 11.1, s=45 21.1, s=64
-// 38.5, s=74 55.1 us), and the walk its `cost` and, with its start and end,
-// 0.4 more.  Block / walk, FP64: s=8 10.6 / 14.9 us, s=30 11.1 / 25.9, s=45
-// 21.1 / 41.5, s=60 34.4 / 41.4, s=76 53.8 / 55.7; walk taken: s=59 31.5 /
-// 27.8, s=74 55.1 / 42.5, s=101 119.8 / 92.3.  FP64_FMA s=64 33.9 / 35.0,
-// mixed s=30 9.8 / 13.7, s=63 25.0 / 26.7.
+// walking kernel's time (8.3 us a plane in FP64), and the walk its `cost` and,
+// with its start and end, 0.4 more.  Block / the fastest walk, us: FP64 s=30 8.6 /
+// 20.3, s=45 17.1 / 31.3, s=60 31.6 / 31.8, s=64 34.0 / 31.8 (whose cycle begins
+// in a launch of 3 us, the block's in the block kernel for 1.6); walk taken: FP64
+// s=101 119.8 / 92.3.
 inline bool block_is_faster(int64_t blocks, int slots, double cost)
 {
    return slots > 0 && (double)blocks < (cost - 0.6) * slots;

@@ -26,13 +26,9 @@ hipError_t launch_widen(const float *src, double *dst, int64_t n, hipStream_t st
 
 // Small fields are copied by a kernel between pinned memory and the device,
 // waited for by its counts: hipMemcpy takes 12 us below 16 KiB and another path
-// above.  Upload and download, hipMemcpy / so: 512 values 12.4 and 12.6 / 8.5 and
-// 8.1 us, 1,728 12.6 and 13.0 / 9.8 and 9.4, 4,096 9.8 and 9.9 / 10.7 and 10.7, 8,000
-// 10.3 and 11.3 / 12.1 and 12.7, 13,824 11.3 and 13.2 / 14.8 and 16.5.  hipMemcpy has
-// to wait for the stream, 9 us after a kernel, so a context copies all of its
-// fields one way (copies_by_kernel): 24 members of 5..24, 11 fields, hipMemcpy
-// 3.50 and 3.70 ms, members of up to 2,048 elements so 3.05 and 3.03, all 2.82 and
-// 2.72.
+// above.  Upload, hipMemcpy / so, us: 512 values 12.4 / 8.5, 1,728 12.6 / 9.8, 4,096
+// 9.8 / 10.7.  hipMemcpy has to wait for the stream, 9 us after a kernel, so a
+// context copies all of its fields one way (copies_by_kernel).
 constexpr int kSmallProblem = 4096, kSmallMembers = 16384; // largest fields
 constexpr int kSmallWave = 128; // values per wave
 constexpr size_t small_copy_bytes(int values) // pinned memory; values a multiple of kSmallWave

@@ -64,7 +64,7 @@ struct Consts {
    int32_t fastEos; // fast_eos_consts(*this), set by the host
 };
 
-// The constants k_eos's fast FP64 EOS repeats assume: e_cut and p_cut
+// The constants k_eos's fast EOS repeats assume (both arithmetics): e_cut and p_cut
 // positive (the values then clamped below by emin and pmin are never -0),
 // emin and pmin not -0 and of magnitude <= 2^100, refdens in [2^-64, 2^64].
 inline bool fast_eos_consts(const Consts &k)

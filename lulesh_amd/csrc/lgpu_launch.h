@@ -35,14 +35,9 @@ constexpr int kEosShare = 4;
 // problem (`repeats` in all), and the larger the launch, within which such
 // waves run beside the others, the more repeats the group has to hold: one per
 // element of the problem for 365,000 elements of the launch (mixed 150,000).
-// One thread / shared, us, 11 regions, FP64 and FP64_FMA: s=8 10 repeats 11.5 /
-// 9.5; s=30 10 12.9 / 10.0, 20 16.4 / 10.8; s=64 10 18.1 / 18.4, 50 34.1 / 32.0; s=81
-// 10 25.7 / 26.8; s=96 10 33.5 / 37.4, 20 43.9 / 44.2, 50 77.8 / 64.0; s=101 10 38.9 /
-// 42.4, 20 51.8 / 50.0, 50 93.8 / 73.1; s=128 20 84.7 / 99.9, 50 151 / 132; 5 regions:
-// s=101 10 51.8 / 50.5, 20 72.7 / 62.7, s=128 20 116 / 123; 21 regions: s=192 30 286 /
-// 333.  Mixed, 16 regions: s=63 10 15.5 / 14.8, 50 28.2 / 21.9; 21 regions: s=101 20
-// 30.2 / 35.1, 50 41.0 / 43.4.  Near the mean (9 for half of the elements): mixed
-// s=63 30.0 / 38.4, s=101 110 / 132.
+// One thread / shared, us: FP64, 11 regions, s=30 of 10 repeats 12.9 / 10.0, s=101 of
+// 10 38.9 / 42.4 and of 50 93.8 / 73.1; mixed, 16 regions, s=63 of 50 28.2 / 21.9, near
+// the mean 30.0 / 38.4.
 inline bool eos_shares(int64_t launchElems, int64_t numElem, const EosGroup &g, double repeats,
                        bool mixed)
 {
@@ -63,10 +58,8 @@ inline void add_eos_slots(std::vector<EosSlot> &slots, const EosGroup &g, bool s
 // k_force, of `blocks` workgroups on `slots` resident ones) instead of
 // k_begin_cycle, a launch of 3.0 to 4.7 us.  Each workgroup then starts up to 1
 // us later, so the gain is gone after a few rounds (4 of k_nodal_block in FP64,
-// otherwise 2).  Launch / first kernel, us a cycle, FP64: s=8 24.6 / 21.5, s=45
-// 37.6 / 36.1, s=55 (2.4 rounds) 46.7 / 45.7, s=64 (3.6) 64.6 / 63.8; FP64_FMA s=64
-// 58.5 / 57.5; mixed s=63 (2.4) 44.5 / 44.9, s=70 (3.4) 52.5 / 55.3; gathers s=64
-// (2) 82.2 / 81.2, s=72 (2.9) 108.6 / 108.3.
+// otherwise 2).  Launch / first kernel, us a cycle: FP64 s=8 24.6 / 21.5, s=64 (3.6
+// rounds) 64.6 / 63.8; mixed s=63 (2.4) 44.5 / 44.9; gathers s=64 (2) 82.2 / 81.2.
 inline bool fold_start(int64_t blocks, int64_t slots, bool fp64Block)
 {
    return blocks <= (fp64Block ? 4 : 2) * slots;
